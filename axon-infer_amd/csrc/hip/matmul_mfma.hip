@@ -18,6 +18,9 @@
 #include "common.h"
 #include "matvec.h"
 
+#include <type_traits>
+#include <utility>
+
 namespace axon_hip {
 
 namespace {
@@ -27,6 +30,7 @@ constexpr int kTileM = 64;  // activation rows per workgroup
 constexpr int kTileN = 64;  // weight rows per workgroup
 
 typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
+typedef int32_t i32x16 __attribute__((ext_vector_type(16)));
 
 template <int T>
 constexpr int block_bytes() {
@@ -445,31 +449,30 @@ __global__ __launch_bounds__(kThreads) void mfma_rows_kernel(MatvecArgs args, Ro
 
 }
 
-// ---- Many activation rows (prefill, mixed passes): 65 rows and more ------------------------
-// A workgroup owns TN weight rows x 64 activation rows; wave w owns activation rows
-// 16w..16w+15 against all TN weight rows, so each MFMA runs once and the wave that ran it folds
-// its four results: per block a lane folds TN/16 x 4 outputs, with one float4 of activation
-// scales and TN/16 weight scales from LDS. The K chunks (kTileChunk blocks) load into registers
-// while the previous chunk computes and expand into aligned int8 in LDS as in mfma_rows_kernel;
-// the scales sit block-major ([block][row], padded) so a lane's four activation scales are one
-// 16-byte read. Every segment of the call is one grid. The per-output order is the scalar
-// table's: block after block, acc += float(sumi) * d_w * d_x (+ m_w * d_x * float(sumx), Q4_1).
+// ---- Few activation rows, wide matrices (batched decode): up to 32 rows ----------------------
+// A workgroup owns TN weight rows x TM = 16 or 32 activation rows, and its four waves split the
+// tile's (activation tile, weight sub-tile) pairs, so each MFMA runs once and the wave that ran it
+// folds its four results: per block a lane reads one float4 of activation scales and its weight
+// scales from LDS. The K chunks (kTileChunk blocks) load into registers while the previous chunk
+// computes and expand into aligned int8 in LDS as in mfma_rows_kernel; the scales sit block-major
+// ([block][row], padded) so a lane's four activation scales are one 16-byte read. Every segment of
+// the call is one grid. The per-output order is the scalar table's: block after block,
+// acc += float(sumi) * d_w * d_x (+ m_w * d_x * float(sumx), Q4_1).
 constexpr uint32_t kTileChunk = 16;
 constexpr uint32_t kTilePitch = kTileChunk * 8 + 4;  // dwords per expanded row
-constexpr uint32_t kTileRows = 64;
 
 template <uint32_t TN>
 __host__ __device__ constexpr uint32_t tile_wp() { return TN + 4; }  // scale pitch, weights
-template <uint32_t TM = kTileRows>
+template <uint32_t TM>
 __host__ __device__ constexpr uint32_t tile_xp() { return TM + 4; }  // scale pitch, activations
 
-template <int T, uint32_t TN, uint32_t TM = kTileRows>
+template <int T, uint32_t TN, uint32_t TM>
 __host__ __device__ constexpr size_t tile_lds() {
   const size_t scales = static_cast<size_t>(kTileChunk) * (tile_wp<TN>() + tile_xp<TM>()) * (T == Q4_1 ? 2 : 1);
   return (static_cast<size_t>(TN + TM) * kTilePitch + scales) * 4;
 }
 
-template <int T, uint32_t TN, bool SWIGLU = false, uint32_t TM = kTileRows>
+template <int T, uint32_t TN, bool SWIGLU, uint32_t TM>
 __global__ __launch_bounds__(kThreads) void mfma_tile_kernel(MatvecArgs args) {
   constexpr int bs = block_bytes<T>();
   constexpr uint32_t KC = kTileChunk, P = kTilePitch;
@@ -477,10 +480,10 @@ __global__ __launch_bounds__(kThreads) void mfma_tile_kernel(MatvecArgs args) {
   constexpr uint32_t NT = TN / 16;                      // weight sub-tiles of the tile
   // The four waves split the tile's (activation tile, weight sub-tile) pairs: with MT
   // activation tiles of 16 rows, wave w takes activation tile w % MT and NTW weight sub-tiles
-  // from (w / MT) * NTW on (all NT when the tile has 64 activation rows).
+  // from (w / MT) * NTW on.
   constexpr uint32_t MT = TM / 16;
   constexpr uint32_t NTW = NT * MT / 4;
-  static_assert(TM == 16 || TM == 32 || TM == 64, "16, 32 or 64 activation rows");
+  static_assert(TM == 16 || TM == 32, "16 or 32 activation rows");
   static_assert(NTW >= 1 && NTW * 4 == NT * MT, "whole sub-tiles per wave");
   constexpr uint32_t WI = TN * KC / kThreads;           // weight items per thread per chunk
   constexpr uint32_t XI = TM * KC / kThreads;           // activation items per thread per chunk
@@ -704,25 +707,20 @@ __global__ __launch_bounds__(kThreads) void mfma_tile_kernel(MatvecArgs args) {
         if (col == 0) *reinterpret_cast<uint16_t*>(blk) = static_cast<uint16_t>(float_to_half_bits(dq));
       }
     };
-    if constexpr (TM == kTileRows) {
+    // A row's gate and up sub-tiles sit on different waves. They meet in LDS ([sub-tile][row][16]
+    // floats; the chunk loop's last barrier freed it), and wave w then takes rows w * TM / 4 ..,
+    // four per pass (one per 16-lane group).
+    float* st = reinterpret_cast<float*>(lds_tile);
 #pragma unroll
-      for (int v = 0; v < 4; ++v) swiglu_row(orow + v, acc[0][v], acc[1][v], acc[2][v], acc[3][v]);
-    } else {
-      // Fewer activation rows: a row's gate and up sub-tiles sit on different waves. They meet
-      // in LDS ([sub-tile][row][16] floats; the chunk loop's last barrier freed it), and wave w
-      // then takes rows w * TM / 4 .., four per pass (one per 16-lane group).
-      float* st = reinterpret_cast<float*>(lds_tile);
+    for (uint32_t j = 0; j < NTW; ++j)
 #pragma unroll
-      for (uint32_t j = 0; j < NTW; ++j)
+      for (int v = 0; v < 4; ++v) st[((j0 + j) * TM + orow + v) * 16 + col] = acc[j][v];
+    __syncthreads();
 #pragma unroll
-        for (int v = 0; v < 4; ++v) st[((j0 + j) * TM + orow + v) * 16 + col] = acc[j][v];
-      __syncthreads();
-#pragma unroll
-      for (uint32_t p = 0; p < TM / 16; ++p) {
-        const uint32_t rr = wave * (TM / 4) + 4 * p + kq;
-        swiglu_row(rr, st[rr * 16 + col], st[(TM + rr) * 16 + col], st[(2 * TM + rr) * 16 + col],
-                   st[(3 * TM + rr) * 16 + col]);
-      }
+    for (uint32_t p = 0; p < TM / 16; ++p) {
+      const uint32_t rr = wave * (TM / 4) + 4 * p + kq;
+      swiglu_row(rr, st[rr * 16 + col], st[(TM + rr) * 16 + col], st[(2 * TM + rr) * 16 + col],
+                 st[(3 * TM + rr) * 16 + col]);
     }
     return;
   }
@@ -741,7 +739,481 @@ __global__ __launch_bounds__(kThreads) void mfma_tile_kernel(MatvecArgs args) {
   }
 }
 
-template <uint32_t TN, uint32_t TM = kTileRows>
+// ---- Many activation rows, wide tiles: 32 x 32 MFMA sums ------------------------------------
+// The same sums and the same per-output expression on v_mfma_i32_32x32x32_i8, which takes one
+// 32-element block of 32 activation rows against 32 weight rows in 14 ns where four 16x16x32 take
+// 34. The 16x16 tiles are bound by LDS (60 % busy, 40 % of that bank conflicts), the expansion of
+// blocks and waits in front of folds; so here
+//   * a wave owns 32 activation rows x 32 WN weight rows: per block it reads its A operand and the
+//     16 activation scales of its lanes once for WN MFMAs, each operand in one 16-byte read;
+//   * blocks are loaded and expanded in pairs: two Q8_0 blocks are 17 dwords and two Q4_0 blocks 9
+//     from a 4-byte boundary, so the first block of a pair is always shifted by 16 bits and the
+//     second never;
+//   * Q4_0 nibbles enter as 16 (q - 8), formed in the byte's high half by a mask and a flipped sign
+//     bit; the sum is then 16 sumi and the scale d_w / 16, both exact;
+//   * the blocks of a chunk are software-pipelined in an order the compiler keeps: a block's MFMAs
+//     are issued before the previous block's folds, and what the folds after those read from LDS
+//     is under way meanwhile.
+// MW of the four waves stack along the activation rows, the others along the weight rows. Where the
+// outputs are too few for that many 32 x 32 tiles (S = 16) a wave owns 16 x 16 WN outputs and the sums
+// are v_mfma_i32_16x16x32_i8's. Q4_0 512 x 16384 x 2048: 99 -> 67 us, with the SwiGLU epilogue 110 ->
+// 74; 128 x 2048 x 8192: 48 -> 31; Q4_1 512 x 5632 x 2048: 62 -> 47. (Raw blocks by LDS-DMA and operands
+// formed by each wave from them, without the expanded copy, ran 83 us: the 4-byte reads of raw rows
+// conflict in LDS.)
+// The scaled block sum fl(float(sumi) * d_w) without the conversion. The MFMA accumulates onto the
+// bits of 1.5 * 2^23, so its result read as a float is 1.5 * 2^23 + sumi exactly (|sumi| <= 2^19),
+// and fma(that, d_w, -1.5 * 2^23 * d_w) is sumi * d_w rounded once: the addend is exact (two bits
+// times an 11-bit half). v_cvt_f32_i32 issues at half the rate of v_fma_f32 here (1.72 against
+// 0.97 ns per SIMD), so a term costs 2.9 instead of 4.6 ns of issue. A zero sum comes out +0 where
+// the product may be -0, which no sum that starts at +0 can tell. A weight scale that is infinite
+// or NaN breaks the cancellation: PLAIN takes the multiply, and a tile that meets such a scale
+// uses it from then on.
+constexpr float kSumBias = 12582912.0f;
+constexpr int32_t kSumBiasBits = 0x4b400000;
+
+template <bool PLAIN>
+__device__ __forceinline__ float scaled_sum(int32_t biased, float dw, float bias_dw) {
+  const float s = __int_as_float(biased);
+  if constexpr (PLAIN) return (s - kSumBias) * dw;
+  else return __builtin_fmaf(s, dw, bias_dw);
+}
+
+__device__ __forceinline__ bool half_not_finite(uint32_t h) { return (h & 0x7c00u) == 0x7c00u; }
+
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_each(F f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F f) { static_for_each(f, std::make_integer_sequence<int, N>{}); }
+
+// The value that lane L of this lane's row of 16 holds.
+template <int L>
+__device__ __forceinline__ float row_lane(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x150 + L, 0xf, 0xf, true));  // row_newbcast
+}
+
+template <int CTRL>
+__device__ __forceinline__ float max_dpp(float x) {
+  return fmaxf(x, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true)));
+}
+
+// The largest of a 16-lane row, in every lane of it: exchanges inside quads, halves and the row.
+__device__ __forceinline__ float row_max(float x) {
+  x = max_dpp<0xb1>(x);       // quad_perm 1,0,3,2
+  x = max_dpp<0x4e>(x);       // quad_perm 2,3,0,1
+  x = max_dpp<0x141>(x);      // row_half_mirror
+  return max_dpp<0x140>(x);   // row_mirror
+}
+
+// The largest of the 32 lanes of a half-wave: of its two rows, which meet by a swizzle (lane ^ 16).
+__device__ __forceinline__ float half_wave_max(float x) {
+  x = row_max(x);
+  return fmaxf(x, __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(x), 0x401f)));
+}
+
+template <int T>
+__host__ __device__ constexpr uint32_t pair_dwords() { return (2 * block_bytes<T>() + 3) / 4; }
+
+template <uint32_t KC>
+__host__ __device__ constexpr uint32_t wide_pitch() { return KC * 8 + 4; }  // dwords per expanded row
+
+template <int T, uint32_t TM, uint32_t TN, uint32_t KC>
+__host__ __device__ constexpr size_t wide_lds() {
+  return (static_cast<size_t>(TN + TM) * wide_pitch<KC>() + static_cast<size_t>(KC) * (TN + TM + 8) * (T == Q4_1 ? 2 : 1)) * 4;
+}
+
+template <int T, uint32_t S, uint32_t MW, uint32_t WN, uint32_t KC, bool SWIGLU = false>
+__global__ __launch_bounds__(kThreads, 2) void mfma_wide_kernel(MatvecArgs args) {
+  constexpr int bs = block_bytes<T>();
+  constexpr uint32_t P = wide_pitch<KC>(), PR = KC / 2;  // PR pairs per row of a chunk
+  constexpr uint32_t NW = 4 / MW, TM = S * MW, TN = S * WN * NW;
+  constexpr uint32_t ND = S * S / 64;  // sums per lane of one MFMA: 16, or 4
+  constexpr uint32_t WP = TN + 4, XP = TM + 4;  // scale pitches
+  constexpr uint32_t WI = TN * PR / kThreads, XI = TM * PR / kThreads;  // pairs per thread per chunk
+  constexpr uint32_t WD = pair_dwords<T>(), XD = pair_dwords<Q8_0>();
+  static_assert(TN * PR % kThreads == 0 && TM * PR % kThreads == 0, "whole pairs per thread");
+  static_assert(S == 32 || S == 16, "32 x 32 or 16 x 16 sums");
+  static_assert(!SWIGLU || (WN * S % 64 == 0 && S % (64 / PR) == 0),
+                "a wave holds gate and up columns of the same whole blocks, and loads rows of one sub-tile at a time");
+
+  extern __shared__ __attribute__((aligned(16))) uint32_t lds_wide[];
+  uint32_t* wa = lds_wide;                            // [TN][P]
+  uint32_t* xa = wa + TN * P;                         // [TM][P]
+  float* wd = reinterpret_cast<float*>(xa + TM * P);  // [KC][WP]
+  float* xd = wd + KC * WP;                           // [KC][XP]
+  float* wmn = xd + KC * XP;                          // [KC][WP] (Q4_1)
+  float* xs = wmn + KC * WP;                          // [KC][XP] (Q4_1): d_x * sumx
+  __shared__ uint32_t plain;  // a weight scale of this tile so far is infinite or NaN
+
+  const uint32_t tid = threadIdx.x;
+  const uint32_t lane = tid & 63;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int s = 0;
+  if (!SWIGLU && args.n_seg > 1 && blockIdx.x >= args.seg[1].wg_begin) s = 1;
+  if (!SWIGLU && args.n_seg > 2 && blockIdx.x >= args.seg[2].wg_begin) s = 2;
+  const MatvecSeg seg = args.seg[s];
+  // SwiGLU: of each wave's WN sub-tiles of S columns the first half are gate rows, the rest the up
+  // rows of the same outputs; the tile's outputs are n0 .. n0 + TN / 2 - 1.
+  constexpr uint32_t TO = SWIGLU ? TN / 2 : TN;
+  const uint32_t n0 = (SWIGLU ? blockIdx.x : blockIdx.x - seg.wg_begin) * TO;
+  const uint32_t m0 = blockIdx.y * TM;
+  const uint32_t nn = min(TO, seg.n_out - n0);
+  const uint32_t mm = min(TM, args.m - m0);
+  const uint32_t nb = args.nb;
+  const uint32_t n_chunks = (nb + KC - 1) / KC;
+  const uint32_t w_pitch = nb * bs, x_pitch = nb * kBytesQ8_0;
+  const __amdgpu_buffer_rsrc_t wsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint8_t*>(seg.w) + static_cast<size_t>(n0) * w_pitch, 0, static_cast<int>(nn * w_pitch),
+      static_cast<int>(kRawBufferWord3));
+  const __amdgpu_buffer_rsrc_t usrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint8_t*>(SWIGLU ? args.seg[1].w : seg.w) + static_cast<size_t>(n0) * w_pitch, 0,
+      static_cast<int>(nn * w_pitch), static_cast<int>(kRawBufferWord3));
+  const __amdgpu_buffer_rsrc_t xsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint8_t*>(args.xq) + static_cast<size_t>(m0) * x_pitch, 0, static_cast<int>(mm * x_pitch),
+      static_cast<int>(kRawBufferWord3));
+
+  struct Raw {
+    uint32_t w[WI][WD];
+    uint32_t x[XI][XD];
+  };
+  // Item k of a thread: pair lane % PR of tile row k * kRowsPer + wave * (64 / PR) + lane / PR
+  // (consecutive lanes, consecutive pairs of a row). Loads past a resource's bytes return zero and
+  // touch nothing (rows past the last, a row's last partial chunk past the end); what a partial
+  // chunk reads of the next row is never folded.
+  constexpr uint32_t kRowsPer = kThreads / PR;
+  const uint32_t irow = wave * (64 / PR) + lane / PR, ipair = lane % PR;
+  auto load = [&](uint32_t c, Raw& r) {
+    const uint32_t p0 = c * PR + ipair;
+#pragma unroll
+    for (uint32_t k = 0; k < WI; ++k) {
+      const uint32_t row = k * kRowsPer + irow;
+      bool upper = false;
+      uint32_t out = row;
+      if constexpr (SWIGLU) {
+        const uint32_t sub = (k * kRowsPer + wave * (64 / PR)) / S;  // uniform in the wave
+        upper = sub % WN >= WN / 2;
+        out = (sub / WN * (WN / 2) + sub % (WN / 2)) * S + row % S;
+      }
+      const uint32_t off = out * w_pitch + p0 * (2 * bs);
+#pragma unroll
+      for (uint32_t d = 0; d < WD; ++d)
+        r.w[k][d] = __builtin_amdgcn_raw_buffer_load_b32(upper ? usrc : wsrc, off + 4 * d, 0, 0);
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < XI; ++k) {
+      const uint32_t off = (k * kRowsPer + irow) * x_pitch + p0 * (2 * kBytesQ8_0);
+#pragma unroll
+      for (uint32_t d = 0; d < XD; ++d) r.x[k][d] = __builtin_amdgcn_raw_buffer_load_b32(xsrc, off + 4 * d, 0, 0);
+    }
+  };
+  if (tid == 0) plain = 0;
+  __syncthreads();
+  // The 8 quant dwords of a Q8_0 pair's block h (its scale: the low half of dword 0, or the high
+  // half of dword 8).
+  auto q8_of = [](const uint32_t (&v)[pair_dwords<Q8_0>()], uint32_t h, uint32_t (&q)[8]) {
+#pragma unroll
+    for (uint32_t j = 0; j < 8; ++j) q[j] = h == 0 ? __builtin_amdgcn_alignbit(v[j + 1], v[j], 16) : v[9 + j];
+  };
+  auto put = [](uint32_t* row, uint32_t b, const uint32_t (&q)[8]) {
+    uint4* dst = reinterpret_cast<uint4*>(row + b * 8);
+    dst[0] = make_uint4(q[0], q[1], q[2], q[3]);
+    dst[1] = make_uint4(q[4], q[5], q[6], q[7]);
+  };
+  auto expand = [&](const Raw& r) {
+    bool odd = false;
+#pragma unroll
+    for (uint32_t k = 0; k < WI; ++k) {
+      const uint32_t row = k * kRowsPer + irow;
+#pragma unroll
+      for (uint32_t h = 0; h < 2; ++h) {
+        const uint32_t b = 2 * ipair + h;
+        const uint32_t(&v)[WD] = r.w[k];
+        uint32_t q[8], sc, mn = 0;
+        if constexpr (T == Q8_0) {
+          q8_of(v, h, q);
+          sc = h == 0 ? v[0] & 0xffffu : v[8] >> 16;
+        } else {
+          uint32_t n4[4];
+          if constexpr (T == Q4_0) {
+            sc = h == 0 ? v[0] & 0xffffu : v[4] >> 16;
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) n4[j] = h == 0 ? __builtin_amdgcn_alignbit(v[j + 1], v[j], 16) : v[5 + j];
+          } else {
+            sc = v[5 * h] & 0xffffu;
+            mn = v[5 * h] >> 16;
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) n4[j] = v[5 * h + 1 + j];
+          }
+#pragma unroll
+          for (uint32_t j = 0; j < 4; ++j) {
+            if constexpr (T == Q4_0) {  // 16 (q - 8) per byte
+              q[j] = ((n4[j] << 4) & 0xf0f0f0f0u) ^ 0x80808080u;
+              q[j + 4] = (n4[j] & 0xf0f0f0f0u) ^ 0x80808080u;
+            } else {
+              q[j] = n4[j] & 0x0f0f0f0fu;
+              q[j + 4] = (n4[j] >> 4) & 0x0f0f0f0fu;
+            }
+          }
+        }
+        put(wa + row * P, b, q);
+        const float dw = half_value(sc);
+        wd[b * WP + row] = T == Q4_0 ? dw * 0.0625f : dw;
+        odd = odd || half_not_finite(sc);
+        if constexpr (T == Q4_1) wmn[b * WP + row] = half_value(mn);
+      }
+    }
+    if (odd) plain = 1;
+#pragma unroll
+    for (uint32_t k = 0; k < XI; ++k) {
+      const uint32_t row = k * kRowsPer + irow;
+#pragma unroll
+      for (uint32_t h = 0; h < 2; ++h) {
+        const uint32_t b = 2 * ipair + h;
+        uint32_t q[8];
+        q8_of(r.x[k], h, q);
+        put(xa + row * P, b, q);
+        const float dx = half_value(h == 0 ? r.x[k][0] & 0xffffu : r.x[k][8] >> 16);
+        xd[b * XP + row] = dx;
+        if constexpr (T == Q4_1) {
+          int32_t sum = 0;
+#pragma unroll
+          for (uint32_t j = 0; j < 8; ++j) sum = __builtin_amdgcn_sdot4(static_cast<int32_t>(q[j]), 0x01010101, sum, false);
+          xs[b * XP + row] = dx * static_cast<float>(sum);  // exact, as in mfma_tile_kernel
+        }
+      }
+    }
+  };
+
+  // Operand and result layout. S = 32: lane l holds elements 16 (l / 32) .. + 15 of row l % 32 of
+  // either operand, and of the sums weight column l % 32, activation rows 8 (v / 4) + 4 (l / 32) +
+  // v % 4. S = 16: elements 8 (l / 16) .. + 7 of row l % 16; column l % 16, rows 4 (l / 16) + v.
+  typedef std::conditional_t<S == 32, i32x4, int64_t> Operand;
+  typedef std::conditional_t<S == 32, i32x16, i32x4> Sum;
+  constexpr uint32_t kOp = S == 32 ? 4 : 2;  // dwords of an operand
+  const uint32_t col = lane % S, part = lane / S;
+  const uint32_t wm = wave % MW, wn = wave / MW;
+  const uint32_t* ap = xa + (wm * S + col) * P + kOp * part;
+  const uint32_t* bp = wa + (wn * WN * S + col) * P + kOp * part;
+  const float* dxp = xd + wm * S + 4 * part;
+  const float* sxp = xs + wm * S + 4 * part;
+  const float* dwp = wd + wn * WN * S + col;
+  const float* mwp = wmn + wn * WN * S + col;
+  auto row_of = [&](uint32_t v) { return wm * S + (S == 32 ? 8 * (v / 4) : 0) + 4 * part + v % 4; };
+  float acc[WN][ND];
+#pragma unroll
+  for (uint32_t j = 0; j < WN; ++j)
+#pragma unroll
+    for (uint32_t v = 0; v < ND; ++v) acc[j][v] = 0.0f;
+  Sum bias;
+#pragma unroll
+  for (uint32_t v = 0; v < ND; ++v) bias[v] = kSumBiasBits;
+
+  struct Operands {
+    Operand a, w[WN];
+  };
+  struct Scales {
+    float dw[WN], mw[WN], dx[ND], sx[ND];
+  };
+  struct Sums {
+    Sum d[WN];
+  };
+  auto fetch = [&](uint32_t b, Operands& o) {
+    o.a = *reinterpret_cast<const Operand*>(ap + b * 8);
+#pragma unroll
+    for (uint32_t j = 0; j < WN; ++j) o.w[j] = *reinterpret_cast<const Operand*>(bp + j * S * P + b * 8);
+  };
+  auto fetch_scales = [&](uint32_t b, Scales& o) {
+#pragma unroll
+    for (uint32_t j = 0; j < WN; ++j) {
+      o.dw[j] = dwp[b * WP + j * S];
+      if constexpr (T == Q4_1) o.mw[j] = mwp[b * WP + j * S];
+    }
+#pragma unroll
+    for (uint32_t g = 0; g < ND / 4; ++g) {
+      const float4 t = *reinterpret_cast<const float4*>(dxp + b * XP + 8 * g);
+      o.dx[4 * g] = t.x;
+      o.dx[4 * g + 1] = t.y;
+      o.dx[4 * g + 2] = t.z;
+      o.dx[4 * g + 3] = t.w;
+      if constexpr (T == Q4_1) {
+        const float4 u = *reinterpret_cast<const float4*>(sxp + b * XP + 8 * g);
+        o.sx[4 * g] = u.x;
+        o.sx[4 * g + 1] = u.y;
+        o.sx[4 * g + 2] = u.z;
+        o.sx[4 * g + 3] = u.w;
+      }
+    }
+  };
+  auto sums = [&](const Operands& o, Sums& d) {
+#pragma unroll
+    for (uint32_t j = 0; j < WN; ++j) {
+      if constexpr (S == 32) d.d[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(o.a, o.w[j], bias, 0, 0, 0);
+      else d.d[j] = __builtin_amdgcn_mfma_i32_16x16x32_i8(o.a, o.w[j], bias, 0, 0, 0);
+    }
+  };
+  auto fold = [&]<bool PLAIN>(const Sums& d, const Scales& o) {
+#pragma unroll
+    for (uint32_t j = 0; j < WN; ++j) {
+      const float dw = o.dw[j], bias_dw = -kSumBias * dw;
+#pragma unroll
+      for (uint32_t v = 0; v < ND; ++v) {
+        const float t = scaled_sum<PLAIN>(d.d[j][v], dw, bias_dw) * o.dx[v];
+        if constexpr (T == Q4_1) acc[j][v] += t + o.mw[j] * o.sx[v];
+        else acc[j][v] += t;
+      }
+    }
+  };
+  // A whole chunk. Block b's sums are in d[b % 2] when its fold begins; the MFMAs of block b + 1 were
+  // issued before it, and block b + 2's operands and block b + 1's scales are read during it.
+  auto whole = [&] {
+    Operands o[2];
+    Scales sc[2];
+    Sums d[2];
+    fetch(0, o[0]);
+    fetch_scales(0, sc[0]);
+    fetch(1, o[1]);
+    sums(o[0], d[0]);
+#pragma unroll
+    for (uint32_t b = 0; b < KC; ++b) {
+      if (b + 1 < KC) sums(o[(b + 1) % 2], d[(b + 1) % 2]);
+      if (b + 2 < KC) fetch(b + 2, o[b % 2]);
+      if (b + 1 < KC) fetch_scales(b + 1, sc[(b + 1) % 2]);
+      __builtin_amdgcn_sched_barrier(0);
+      fold.template operator()<false>(d[b % 2], sc[b % 2]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  auto block = [&]<bool PLAIN>(uint32_t b) {
+    Operands o;
+    Scales sc;
+    Sums d;
+    fetch(b, o);
+    fetch_scales(b, sc);
+    sums(o, d);
+    fold.template operator()<PLAIN>(d, sc);
+  };
+
+  Raw r;
+  load(0, r);
+  for (uint32_t c = 0; c < n_chunks; ++c) {
+    const uint32_t cb = min(KC, nb - c * KC);  // even: a row is whole pairs
+    expand(r);
+    __syncthreads();
+    if (c + 1 < n_chunks) load(c + 1, r);
+    asm volatile("" : "+v"(bias));  // kept in registers
+    if (__builtin_amdgcn_readfirstlane(plain) != 0) {
+#pragma unroll 1
+      for (uint32_t b = 0; b < cb; ++b) block.template operator()<true>(b);
+    } else if (cb == KC) {
+      whole();
+    } else {
+#pragma unroll 1
+      for (uint32_t b = 0; b < cb; ++b) block.template operator()<false>(b);
+    }
+    __syncthreads();
+  }
+
+  if constexpr (SWIGLU) {
+    // silu(gate) * up as silu_mul_kernel forms it, then each row's 32 outputs as one Q8_0 block
+    // (quantize_block_lanes' steps): a half-wave holds a block (S = 32), or a row of 16 lanes two
+    // values of it each. A lane's ND rows go side by side, with nothing conditional before the
+    // stores, and the two divisions of a block run once for ND blocks: lane i of a 16-lane row takes
+    // block i and hands 1 / d back by a row broadcast. (Row by row, the epilogue of 512 x 16384 took
+    // 21 of 88 us, of which this left 7.)
+    constexpr uint32_t kY = 32 / S;  // a lane's values of a block
+    uint64_t* tab = reinterpret_cast<uint64_t*>(lds_wide);  // the chunk loop's last barrier freed it
+    if (tid < 32) tab[tid] = kExp2Tab[tid];
+    __syncthreads();
+    const size_t row_blocks = seg.n_out / kQK;
+#pragma unroll
+    for (uint32_t j = 0; j < WN / 2; j += kY) {
+      const uint32_t n = (wn * (WN / 2) + j) * S;
+      if (n >= nn) continue;
+      float y[ND][kY], amax = 0.0f;
+#pragma unroll
+      for (uint32_t v = 0; v < ND; ++v) {
+        float m = 0.0f;
+#pragma unroll
+        for (uint32_t k = 0; k < kY; ++k) {
+          const float g = acc[j + k][v];
+          y[v][k] = g / (1.0f + exp_libm_from(-g, tab)) * acc[j + k + WN / 2][v];
+          m = fmaxf(m, fabsf(y[v][k]));
+        }
+        m = S == 32 ? half_wave_max(m) : row_max(m);
+        amax = (lane & 15u) == v ? m : amax;
+      }
+      const float d = amax / 127.0f;
+      const float id = d != 0.0f ? 1.0f / d : 0.0f;
+      const uint32_t dh = float_to_half_bits(d);
+      static_for<ND>([&](auto vc) {
+        constexpr uint32_t v = vc.value;
+        const uint32_t rr = row_of(v);
+        const uint32_t dv = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(dh), 0x150 + v, 0xf, 0xf, true));
+        uint8_t* blk = args.outq + (static_cast<size_t>(m0 + rr) * row_blocks + (n0 + n) / kQK) * kBytesQ8_0;
+        if (rr < mm && col == 0) *reinterpret_cast<uint16_t*>(blk) = static_cast<uint16_t>(dv);
+#pragma unroll
+        for (uint32_t k = 0; k < kY; ++k) {
+          const int32_t q = static_cast<int32_t>(roundf(y[v][k] * row_lane<v>(id)));
+          const int32_t q_next = __builtin_amdgcn_update_dpp(0, q, 0xf5, 0xf, 0xf, true);  // quad_perm 1,1,3,3
+          if (rr < mm) {
+            if (seg.y != nullptr) seg.y[static_cast<size_t>(m0 + rr) * seg.y_stride + n0 + n + k * S + col] = y[v][k];
+            if ((col & 1u) == 0)
+              *reinterpret_cast<uint16_t*>(blk + 2 + k * S + col) = static_cast<uint16_t>((q & 0xff) | ((q_next & 0xff) << 8));
+          }
+        }
+      });
+    }
+    return;
+  }
+#pragma unroll
+  for (uint32_t j = 0; j < WN; ++j) {
+    const uint32_t n = (wn * WN + j) * S + col;
+    if (n < nn) {
+#pragma unroll
+      for (uint32_t v = 0; v < ND; ++v) {
+        const uint32_t rr = row_of(v);
+        if (rr < mm) {
+          float* y = seg.y + static_cast<size_t>(m0 + rr) * seg.y_stride + n0 + n;
+          *y = args.accumulate ? *y + acc[j][v] : acc[j][v];
+        }
+      }
+    }
+  }
+}
+
+template <uint32_t S, uint32_t MW, uint32_t WN, uint32_t KC, bool SWIGLU = false>
+int wide_launch(int type, MatvecArgs& a) {
+  constexpr uint32_t TM = S * MW, TN = S * WN * (4 / MW), TO = SWIGLU ? TN / 2 : TN;
+  uint32_t wg = 0;
+  for (int s = 0; s < (SWIGLU ? 1 : a.n_seg); ++s) {
+    a.seg[s].wg_begin = wg;
+    wg += static_cast<uint32_t>(ceil_div(a.seg[s].n_out, TO));
+  }
+  const dim3 grid(wg, static_cast<uint32_t>(ceil_div(a.m, TM)));
+  static const bool granted = [] {
+    bool ok = true;
+    auto grant = [&](auto kernel, size_t lds) {
+      if (lds > 65536)
+        ok = ok && hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       static_cast<int>(lds)) == hipSuccess;
+    };
+    grant(mfma_wide_kernel<Q8_0, S, MW, WN, KC, SWIGLU>, wide_lds<Q8_0, TM, TN, KC>());
+    grant(mfma_wide_kernel<Q4_0, S, MW, WN, KC, SWIGLU>, wide_lds<Q4_0, TM, TN, KC>());
+    grant(mfma_wide_kernel<Q4_1, S, MW, WN, KC, SWIGLU>, wide_lds<Q4_1, TM, TN, KC>());
+    return ok;
+  }();
+  if (!granted) return fail(kUnsupported, "matmul wide: the LDS grant was refused");
+  switch (type) {
+  case Q8_0: launch(mfma_wide_kernel<Q8_0, S, MW, WN, KC, SWIGLU>, grid, dim3(kThreads), wide_lds<Q8_0, TM, TN, KC>(), a); break;
+  case Q4_0: launch(mfma_wide_kernel<Q4_0, S, MW, WN, KC, SWIGLU>, grid, dim3(kThreads), wide_lds<Q4_0, TM, TN, KC>(), a); break;
+  case Q4_1: launch(mfma_wide_kernel<Q4_1, S, MW, WN, KC, SWIGLU>, grid, dim3(kThreads), wide_lds<Q4_1, TM, TN, KC>(), a); break;
+  default: return fail(kUnsupported, "matmul wide: weight type %d", type);
+  }
+  return check_launch("mfma_wide");
+}
+
+template <uint32_t TN, uint32_t TM>
 int tile_launch(int type, MatvecArgs& a) {
   uint32_t wg = 0;
   for (int s = 0; s < a.n_seg; ++s) {
@@ -850,6 +1322,7 @@ bool matmul_q8_rows_fits(int type, const MatvecArgs& a, bool many_rows) {
 }
 
 constexpr uint32_t kDecodeTileWg = 256;  // workgroups a decode matrix needs for the tile kernel
+constexpr uint32_t kWideMinBlocks = 48;  // blocks per row from which the largest tiles pay
 
 // From 128 tiles of 64 weight rows (33..64 rows, Q4_0): 8192 x 2048 24.4 -> 15.8 us, 9728 x 896
 // 20.7 -> 10.3, 16384 x 2048 46.0 -> 20.7; at 48 tiles and fewer the rows kernel stays ahead.
@@ -899,17 +1372,34 @@ int matmul_q8_swiglu_launch(int type, MatvecArgs& a) {
     return fail(kUnsupported, "matmul swiglu: %u outputs give too few workgroups for %u rows", a.seg[0].n_out, a.m);
   if (a.m <= 16) return swiglu_launch<16>(type, a);
   if (a.m <= 32) return swiglu_launch<32>(type, a);
-  return swiglu_launch<kTileRows>(type, a);
+  // 64 x 64-output tiles of 32 x 32 sums where they are two workgroups per CU, else 64 x 32 outputs
+  // of 16 x 16 sums (Q4_0 2048 -> 8192: 512 rows 74 / 81 us, 200 rows 39 / 48, 128 rows 33 / 27);
+  // short rows too, whose epilogues weigh more (896 -> 4864 at 575 rows 36 / 33).
+  const uint64_t wide = static_cast<uint64_t>(ceil_div(a.seg[0].n_out, 64)) * ceil_div(a.m, 64u);
+  if (wide >= 512 && a.nb >= kWideMinBlocks) return wide_launch<32, 2, 2, 8, true>(type, a);
+  return wide_launch<16, 4, 4, 8, true>(type, a);
 }
 
+// The tile by how many workgroups it gives (two fit a CU): the largest that still fills the chip.
+// Measured at Q4_0, K = 2048, us: 64 x 128 / 64 x 64 tiles of 32 x 32 sums, 32 x 64 / 32 x 32 tiles of
+// 16 x 16 sums (the 16 x 16 kernel these replaced in brackets):
+//   512 x 16384  67 / 72 / 115 / 118 (99)     256 x 5632  29 / 23 / 26 / 27 (30)
+//   512 x 5632   35 / 31 / 44 / 45 (49)       512 x 2048  29 / 20 / 17 / 20 (19)
+//   512 x 3072   29 / 23 / 26 / 27 (29)       128 x 2048  28 / 19 / 13 / 10 (15)
+// Rows of fewer than kWideMinBlocks blocks keep to the smaller tile (896 x 9728 at 512 rows 31 / 25).
 int matmul_q8_tile_launch(int type, MatvecArgs& a) {
   if (!matmul_q8_rows_fits(type, a, true)) return fail(kUnsupported, "matmul tile: shape or alignment");
-  // 64-row weight tiles when they give the chip a few workgroups per CU, else 32-row tiles.
-  uint32_t wg64 = 0;
-  for (int s = 0; s < a.n_seg; ++s) wg64 += static_cast<uint32_t>(ceil_div(a.seg[s].n_out, 64));
-  const uint64_t tiles64 = static_cast<uint64_t>(wg64) * ceil_div(a.m, kTileRows);
-  if (tiles64 >= 768) return tile_launch<64>(type, a);
-  return tile_launch<32>(type, a);
+  auto workgroups = [&](uint32_t tm, uint32_t tn) {
+    uint64_t n = 0;
+    for (int s = 0; s < a.n_seg; ++s) n += ceil_div(a.seg[s].n_out, tn);
+    return n * ceil_div(a.m, tm);
+  };
+  // 128 weight rows behind one buffer descriptor, whose size is 31 bits.
+  const bool sized = static_cast<uint64_t>(a.nb) * kBytesQ8_0 * 128 < (uint64_t(1) << 31);
+  if (workgroups(64, 128) >= 512 && a.nb >= kWideMinBlocks && sized) return wide_launch<32, 2, 2, 8>(type, a);
+  if (workgroups(64, 64) >= 320) return wide_launch<32, 2, 1, 8>(type, a);
+  if (workgroups(32, 64) >= 512) return wide_launch<16, 2, 2, 16>(type, a);
+  return wide_launch<16, 2, 1, 16>(type, a);
 }
 
 int matmul_q8_rows_launch(int type, MatvecArgs& a) {

@@ -106,8 +106,8 @@ constexpr uint32_t kRowsMaxM = 64;
 // many_rows: the prefill tile kernel's bounds (any row count) instead of 1..kRowsMaxM.
 bool matmul_q8_rows_fits(int type, const MatvecArgs& a, bool many_rows = false);
 int matmul_q8_rows_launch(int type, MatvecArgs& a);
-// int8 MFMA for 65 and more activation rows (prefill, mixed passes): TN x 64 tiles, every
-// segment in one grid, the same per-output order.
+// int8 MFMA for 65 and more activation rows (prefill, mixed passes): tiles of 32 x 32 or 16 x 16
+// sums chosen by the workgroups they give, every segment in one grid, the same per-output order.
 int matmul_q8_tile_launch(int type, MatvecArgs& a);
 // 33..64 rows on matrices of at least 128 tiles of 64 weight rows: the tile kernel reads the
 // weights once where the few-rows kernel's 16-row tiles read them up to four times.
