@@ -33,6 +33,8 @@ constexpr uint32_t kVMaxItems = kVTile * 128 / 4 / kThreads;  // 4-float items p
 constexpr uint32_t kBlockMinWorkgroups = 512;
 constexpr size_t kBlockMaxLds = 80 * 1024;
 constexpr int kBlockWaves = 3;  // waves per SIMD the blocked kernel's registers allow
+// The tiled many-row kernel: only while its blocks leave a workgroup per CU.
+constexpr uint32_t kTileMinWorkgroups = 256;
 
 __host__ __device__ inline uint32_t round4(uint32_t v) { return (v + 3) & ~3u; }
 __host__ __device__ inline size_t vtile_bytes(uint32_t hd) { return static_cast<size_t>(hd) * kVPitch * 4; }
@@ -711,6 +713,470 @@ bool launch_block(const AttnArgs& a, uint32_t n_rows) {
   case 4: return launch_block_g<4>(a, n_rows);
   case 7: return launch_block_g<7>(a, n_rows);
   case 8: return launch_block_g<8>(a, n_rows);
+  default: return false;
+  }
+}
+
+// ---- Many-row launches, products on the matrix cores ----------------------------------------
+// attention_tile_kernel<F16, G, R>: one workgroup per (R consecutive query rows, kv head) for kv
+// groups of G = 4 or 8 query heads of 64 dims; its G R (row, head) pairs go four to a wave. The
+// products are formed on the matrix cores, by v_mfma_f32_4x4x1 with a zero addend: sixteen 4 x 4
+// outer products, four pairs against 64 positions (scores) or 64 dims (values), each element the
+// product of two floats rounded once, as the scalar table's is (a zero product comes out +0, which
+// no sum that starts at +0 can tell); the adds then follow on the vector ALU in the scalar table's
+// order, lane = position over d, then lane = dim over positions. What that buys is not the
+// multiplies (an MFMA costs about what four of them do) but their operands: a broadcast of pairs is
+// an operand modifier, where a multiply took it from LDS (one 16-byte read per pair and 4 positions)
+// or from a scalar register (v_mul_f32 with one issues at half rate). So LDS holds little but the
+// scores, and a workgroup keeps 32 pairs at up to 1088 positions, or 16 at 2176, where the blocked
+// kernel above falls back to one row at a time from about 1000.
+//   scores   K tiles of 64 positions x 32 dims go through a ring of three 8 KB stages by LDS-DMA
+//            (16-byte chunks XOR-swizzled, so that the lanes' row reads spread over the banks);
+//   softmax  each wave its own four pairs: max, exp, the fused kernel's 256-thread double-sum tree
+//            (lane l carries the partial sums of threads l, l + 64, l + 128, l + 192); the factor
+//            1 / sum is applied as the mix reads the probabilities;
+//   mix      V tiles of 32 positions through the same ring.
+// Rows that do not share one 16-byte-aligned K/V span (the decode rows of a ragged batch) load K and
+// V straight from memory, each wave its own. Blocks are dispatched from the last rows down: in a
+// prefill those see the most positions.
+// Rows of 32 / 8 heads, us before -> now: 512 behind 512 positions 364 -> 135 (of which 56 with no
+// arithmetic at all: staging, barriers, the wave reductions), 512 with no past 80 -> 61, 512 behind 1500
+// 1034 -> 511, 256 behind 700 99 -> 82; a 512-row chunk with 63 decode rows 285 -> 212.
+constexpr uint32_t kStagePos = 64;    // positions of a K stage (by 32 dims)
+constexpr uint32_t kStageV = 32;      // positions of a V stage (by 64 dims)
+constexpr uint32_t kStages = 3;
+template <bool F16>
+__host__ __device__ constexpr uint32_t stage_bytes_of() { return F16 ? 4096 : 8192; }
+
+// Floats per pair: whole K tiles, and 16 more so that four pairs' 16 positions hit distinct banks.
+__host__ __device__ inline uint32_t tile_pitch(uint32_t max_vis) { return ((max_vis + 63) & ~63u) + 16; }
+
+template <uint32_t G, uint32_t R>
+__host__ __device__ constexpr uint32_t tile_waves() { return (G * R + 3) / 4; }
+
+template <bool F16, uint32_t G, uint32_t R>
+__host__ __device__ inline size_t tile_lds(uint32_t max_vis) {
+  return kStages * stage_bytes_of<F16>() + static_cast<size_t>(tile_waves<G, R>()) * 4 * tile_pitch(max_vis) * 4;
+}
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// Sixteen 4 x 4 outer products: rows the four values that block K of a holds (lanes 4 K .. 4 K + 3),
+// columns the four lanes of each block of b. Lane l's element v: a[4 K + v] * b[l].
+template <int K>
+__device__ __forceinline__ f32x4 outer4(float a, float b) {
+  const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, zero, 4, K, 0);
+}
+
+// Keeps N outer products and their 4 N adds interleaved, the products two ahead of their adds (left
+// to itself the compiler puts each product right before its adds and waits for it).
+template <int N>
+__device__ __forceinline__ void products_ahead() {
+  __builtin_amdgcn_sched_group_barrier(0x8, 2, 0);
+#pragma unroll
+  for (int i = 0; i < N - 2; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x2, 4, 0);
+  }
+  __builtin_amdgcn_sched_group_barrier(0x2, 8, 0);
+}
+
+template <int I, int N, typename F>
+__device__ __forceinline__ void for_each_index(F f) {
+  if constexpr (I < N) {
+    f.template operator()<I>();
+    for_each_index<I + 1, N>(f);
+  }
+}
+
+template <bool F16, uint32_t G, uint32_t R>
+__global__ __launch_bounds__((64 * tile_waves<G, R>()), 2) void attention_tile_kernel(AttnArgs a, uint32_t n_rows) {
+  constexpr uint32_t kPairs = G * R, W = tile_waves<G, R>();
+  constexpr uint32_t es = F16 ? 2 : 4;
+  constexpr uint32_t kStage = stage_bytes_of<F16>();
+  constexpr uint32_t kCopies = kStage / 1024;  // 1 KB copies per stage
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds_tile[];
+  __shared__ uint64_t exp_tab[32];
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t g = blockIdx.x % a.n_kv;
+  const uint32_t n_blocks = (n_rows + R - 1) / R;
+  const uint32_t r0 = (n_blocks - 1 - blockIdx.x / a.n_kv) * R;
+  const uint32_t pitch = tile_pitch(a.max_vis);
+  float* sc = reinterpret_cast<float*>(lds_tile + kStages * kStage) + wave * 4 * pitch;  // this wave's four pairs
+  for (uint32_t i = tid; i < 32; i += 64 * W) exp_tab[i] = kExp2Tab[i];
+
+  // Each row's span and positions (0 for a row past the launch).
+  int64_t k_off[R], v_off[R];
+  uint32_t nv[R], nmax = 0;
+  bool shared = true;
+  const uintptr_t base = reinterpret_cast<uintptr_t>(a.kv);
+#pragma unroll
+  for (uint32_t i = 0; i < R; ++i) {
+    const uint32_t r = min(r0 + i, n_rows - 1);
+    k_off[i] = (a.k_off != nullptr ? a.k_off[r] : 0) + a.k_off_c;
+    v_off[i] = (a.v_off != nullptr ? a.v_off[r] : 0) + a.v_off_c;
+    nv[i] = r0 + i < n_rows
+                ? (a.n_vis != nullptr ? static_cast<uint32_t>(a.n_vis[r]) : static_cast<uint32_t>(a.n_past) + r + 1)
+                : 0;
+    nmax = max(nmax, nv[i]);
+    if (i > 0 && nv[i] > 0) shared = shared && k_off[i] == k_off[0] && v_off[i] == v_off[0];
+  }
+  auto aligned = [&](int64_t off) { return ((base + static_cast<uintptr_t>(off) * es) & 15u) == 0; };
+  shared = shared && aligned(k_off[0]) && aligned(v_off[0]);
+
+  // Pair 4 wave + v of this wave: its row within the block (R for none) and its positions.
+  uint32_t prow[4], pvis[4], wmax = 0;
+  uint32_t wmin = 0xffffffffu;  // positions that all of the wave's pairs see
+#pragma unroll
+  for (uint32_t v = 0; v < 4; ++v) {
+    const uint32_t pr = 4 * wave + v;
+    prow[v] = pr < kPairs ? pr / G : R;
+    pvis[v] = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < R; ++i) pvis[v] = prow[v] == i ? nv[i] : pvis[v];
+    wmax = max(wmax, pvis[v]);
+    if (pvis[v] > 0) wmin = min(wmin, pvis[v]);
+  }
+
+  const uint32_t ring = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(as_lds(lds_tile)));
+  const size_t kv_row = static_cast<size_t>(a.n_kv) * 64;
+  const uint32_t row_bytes = static_cast<uint32_t>(kv_row * es);
+  const uint32_t my_copies = kCopies > wave ? (kCopies - wave + W - 1) / W : 0;  // per stage
+  auto span = [&](int64_t off) {
+    return raw_buffer_words(static_cast<const uint8_t*>(a.kv) + (off + static_cast<int64_t>(g) * 64) * es,
+                            static_cast<uint32_t>((static_cast<size_t>(max(nmax, 1u) - 1) * kv_row + 64) * es));
+  };
+  // K stage s: positions 64 (s / 2) .. + 63, dims 32 (s % 2) .. + 31; a row is 128 bytes (64 in fp16)
+  // whose 16-byte chunk c sits in slot c ^ swizzle(row). Positions past the last repeat it.
+  constexpr uint32_t kChunks = 32 * es / 16, kRowsPerCopy = 64 / kChunks;
+  auto swizzle = [](uint32_t row) { return F16 ? (row >> 2) & 3u : (row >> 1) & 7u; };
+  auto copy_k = [&](RsrcWords src, uint32_t s) {
+    const uint32_t dst = ring + (s % kStages) * kStage;
+    for (uint32_t i = wave; i < kCopies; i += W) {
+      const uint32_t row = kRowsPerCopy * i + lane / kChunks;
+      const uint32_t pos = min(kStagePos * (s >> 1) + row, nmax - 1);
+      const uint32_t chunk = (lane % kChunks) ^ swizzle(row);
+      lds_dma16(src, pos * row_bytes + (s & 1) * 32 * es + chunk * 16, dst + i * 1024);
+    }
+  };
+  // V stage t: positions 32 t .. + 31, a row after another.
+  constexpr uint32_t kVChunks = 64 * es / 16, kVRows = 64 / kVChunks;
+  auto copy_v = [&](RsrcWords src, uint32_t t) {
+    const uint32_t dst = ring + (t % kStages) * kStage;
+    for (uint32_t i = wave; i < kCopies; i += W) {
+      const uint32_t pos = min(kStageV * t + kVRows * i + lane / kVChunks, nmax - 1);
+      lds_dma16(src, pos * row_bytes + (lane % kVChunks) * 16, dst + i * 1024);
+    }
+  };
+
+  // This lane's part of the pairs' queries: lane 4 b + i of register k holds dim 16 k + b of pair i.
+  float qa[4];
+  {
+    const uint32_t pr = min(4 * wave + (lane & 3u), kPairs - 1);
+    const uint32_t r = min(r0 + pr / G, n_rows - 1);
+    const float* q = a.q + static_cast<size_t>(r) * a.q_stride + static_cast<size_t>(g * G + pr % G) * 64 + (lane >> 2);
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) qa[k] = q[16 * k];
+  }
+
+  // Scores of 64 positions against the wave's pairs: half the dims at a time, in order.
+  float m[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+  f32x4 dot = {0.0f, 0.0f, 0.0f, 0.0f};
+  auto add_half = [&]<int HALF>(const float (&kr)[32]) {
+    f32x4 p[32];
+    for_each_index<0, 32>([&]<int D>() { p[D] = outer4<D % 16>(qa[2 * HALF + D / 16], kr[D]); });
+#pragma unroll
+    for (int d = 0; d < 32; ++d)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) dot[v] += p[d][v];
+    products_ahead<32>();
+  };
+  auto store_scores = [&](uint32_t j0, uint32_t only) {  // only: the row whose pairs are stored, or R for all
+    const uint32_t j = j0 + lane;
+#pragma unroll
+    for (uint32_t v = 0; v < 4; ++v) {
+      if (only == R || prow[v] == only) {
+        const float x = a.scale * dot[v];
+        sc[v * pitch + j] = x;
+        if (j < pvis[v]) m[v] = fmaxf(m[v], x);
+      }
+      dot[v] = 0.0f;
+    }
+  };
+  // 16 positions from j0 on of the value mix: pa holds the probabilities (lane 4 b + i: pair i, position
+  // j0 + b), vr this lane's dim of each position.
+  float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  auto mix16 = [&]<bool WHOLE>(float pa, const float (&vr)[16], uint32_t j0, uint32_t only) {
+    f32x4 p[16];
+    for_each_index<0, 16>([&]<int J>() { p[J] = outer4<J>(pa, vr[J]); });
+    if constexpr (WHOLE) {
+#pragma unroll
+      for (int j = 0; j < 16; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) acc[v] += p[j][v];
+      products_ahead<16>();
+    } else {
+#pragma unroll
+      for (uint32_t v = 0; v < 4; ++v) {
+        const uint32_t end = only == R || prow[v] == only ? pvis[v] : 0;
+        const uint32_t n = end > j0 ? end - j0 : 0;
+#pragma unroll
+        for (uint32_t j = 0; j < 16; ++j) acc[v] = j < n ? acc[v] + p[j][v] : acc[v];
+      }
+    }
+  };
+
+  RsrcWords vsrc{};
+  if (shared && nmax > 0) {
+    const RsrcWords ksrc = span(k_off[0]);
+    vsrc = span(v_off[0]);
+    const uint32_t n_stages = 2 * ((nmax + kStagePos - 1) / kStagePos);
+    copy_k(ksrc, 0);
+    copy_k(ksrc, 1);
+    for (uint32_t s = 0; s < n_stages; s += 2) {
+      auto half = [&]<int HALF>() {
+        const uint32_t st = s + HALF;
+        wait_vm_upto(st + 1 < n_stages ? my_copies : 0);
+        __syncthreads();  // everyone's copies of this stage; the one before the last has been read
+        if (st + 2 < n_stages) copy_k(ksrc, st + 2);
+        if (kStagePos * (s >> 1) >= wmax) return;
+        const uint4* row = reinterpret_cast<const uint4*>(lds_tile + (st % kStages) * kStage) + lane * kChunks;
+        const uint32_t sw = swizzle(lane);
+        float kr[32];
+#pragma unroll
+        for (uint32_t c = 0; c < kChunks; ++c) {
+          const uint4 u = row[c ^ sw];
+          const uint32_t w4[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+          for (uint32_t k = 0; k < 4; ++k) {
+            if constexpr (F16) {
+              kr[8 * c + 2 * k] = half_value(w4[k] & 0xffffu);
+              kr[8 * c + 2 * k + 1] = half_value(w4[k] >> 16);
+            } else {
+              kr[4 * c + k] = __uint_as_float(w4[k]);
+            }
+          }
+        }
+        add_half.template operator()<HALF>(kr);
+        if constexpr (HALF == 1) store_scores(kStagePos * (s >> 1), R);
+      };
+      half.template operator()<0>();
+      half.template operator()<1>();
+    }
+    __syncthreads();  // the ring is free for V
+    copy_v(vsrc, 0);
+    if (kStageV < nmax) copy_v(vsrc, 1);
+  } else {
+    __syncthreads();  // exp_tab is written
+    for (uint32_t i = 0; i < R; ++i) {
+      bool mine = false;
+      int64_t off = 0;
+      uint32_t n = 0;
+#pragma unroll
+      for (uint32_t v = 0; v < 4; ++v) mine = mine || prow[v] == i;
+#pragma unroll
+      for (uint32_t k = 0; k < R; ++k) {
+        off = k == i ? k_off[k] : off;
+        n = k == i ? nv[k] : n;
+      }
+      if (!mine) continue;
+      const bool vec = aligned(off);
+      for (uint32_t j0 = 0; j0 < n; j0 += 64) {
+        const size_t e = static_cast<size_t>(off) + static_cast<size_t>(min(j0 + lane, n - 1)) * kv_row + static_cast<size_t>(g) * 64;
+        auto half = [&]<int HALF>() {
+          float kr[32];
+          if (!vec) {
+#pragma unroll
+            for (uint32_t d = 0; d < 32; ++d) kr[d] = kv_at<F16>(a.kv, e + 32 * HALF + d);
+          } else {
+            const uint4* row = reinterpret_cast<const uint4*>(static_cast<const uint8_t*>(a.kv) + (e + 32 * HALF) * es);
+#pragma unroll
+            for (uint32_t c = 0; c < kChunks; ++c) {
+              const uint4 u = row[c];
+              const uint32_t w4[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+              for (uint32_t k = 0; k < 4; ++k) {
+                if constexpr (F16) {
+                  kr[8 * c + 2 * k] = half_value(w4[k] & 0xffffu);
+                  kr[8 * c + 2 * k + 1] = half_value(w4[k] >> 16);
+                } else {
+                  kr[4 * c + k] = __uint_as_float(w4[k]);
+                }
+              }
+            }
+          }
+          add_half.template operator()<HALF>(kr);
+        };
+        half.template operator()<0>();
+        half.template operator()<1>();
+        store_scores(j0, i);
+      }
+    }
+  }
+
+  // Softmax of the wave's pairs, side by side.
+  float inv[4];
+  {
+#pragma unroll
+    for (uint32_t v = 0; v < 4; ++v) m[v] = wave_max(m[v]);
+    double part[4][4];
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+#pragma unroll
+      for (uint32_t v = 0; v < 4; ++v) part[w][v] = 0.0;
+    // 64 positions of the four pairs at a time, without a branch: a position past a pair's own takes
+    // the exponential of 0 (its score may be anything), adds an exact zero to the sum, and what it
+    // stores is never added by the mix.
+    auto exps = [&](uint32_t j0, double (&p)[4]) {
+      float x[4];
+#pragma unroll
+      for (uint32_t v = 0; v < 4; ++v) x[v] = sc[v * pitch + j0 + lane];
+#pragma unroll
+      for (uint32_t v = 0; v < 4; ++v) x[v] = exp_libm_from(j0 + lane < pvis[v] ? x[v] - m[v] : 0.0f, exp_tab);
+#pragma unroll
+      for (uint32_t v = 0; v < 4; ++v) {
+        sc[v * pitch + j0 + lane] = x[v];
+        p[v] += static_cast<double>(j0 + lane < pvis[v] ? x[v] : 0.0f);
+      }
+    };
+    for (uint32_t j0 = 0; j0 < wmax; j0 += 256) {
+#pragma unroll
+      for (int w = 0; w < 4; ++w)
+        if (j0 + 64 * w < wmax) exps(j0 + 64 * w, part[w]);
+    }
+#pragma unroll
+    for (uint32_t v = 0; v < 4; ++v) {
+      double sum = 0.0;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) sum += wave_sum(part[w][v]);
+      inv[v] = static_cast<float>(1.0 / sum);
+    }
+  }
+  const uint32_t pi = lane & 3u;
+  const float inv_lane = pi == 0 ? inv[0] : pi == 1 ? inv[1] : pi == 2 ? inv[2] : inv[3];
+  const float* pp = sc + pi * pitch + (lane >> 2);
+
+  // Value mix, positions in order.
+  if (shared && nmax > 0) {
+    const uint32_t n_tiles = (nmax + kStageV - 1) / kStageV;
+    for (uint32_t t = 0; t < n_tiles; ++t) {
+      wait_vm_upto(t + 1 < n_tiles ? my_copies : 0);
+      __syncthreads();
+      if (t + 2 < n_tiles) copy_v(vsrc, t + 2);
+      const uint8_t* vt = lds_tile + (t % kStages) * kStage;
+#pragma unroll
+      for (uint32_t u = 0; u < 2; ++u) {
+        const uint32_t j0 = kStageV * t + 16 * u;
+        if (j0 >= wmax) continue;
+        const float pa = pp[j0] * inv_lane;
+        float vr[16];
+#pragma unroll
+        for (uint32_t j = 0; j < 16; ++j) {
+          if constexpr (F16) vr[j] = half_value(reinterpret_cast<const uint16_t*>(vt)[(16 * u + j) * 64 + lane]);
+          else vr[j] = reinterpret_cast<const float*>(vt)[(16 * u + j) * 64 + lane];
+        }
+        if (j0 + 16 <= wmin) mix16.template operator()<true>(pa, vr, j0, R);
+        else mix16.template operator()<false>(pa, vr, j0, R);
+      }
+    }
+  } else {
+    for (uint32_t i = 0; i < R; ++i) {
+      bool mine = false;
+      int64_t off = 0;
+      uint32_t n = 0;
+#pragma unroll
+      for (uint32_t v = 0; v < 4; ++v) mine = mine || prow[v] == i;
+#pragma unroll
+      for (uint32_t k = 0; k < R; ++k) {
+        off = k == i ? v_off[k] : off;
+        n = k == i ? nv[k] : n;
+      }
+      if (!mine) continue;
+      const size_t e = static_cast<size_t>(off) + static_cast<size_t>(g) * 64 + lane;
+      float vr[16], vn[16];
+      auto get = [&](uint32_t j0, float (&v)[16]) {
+#pragma unroll
+        for (uint32_t j = 0; j < 16; ++j) v[j] = kv_at<F16>(a.kv, e + static_cast<size_t>(min(j0 + j, n - 1)) * kv_row);
+      };
+      if (n > 0) get(0, vr);
+      for (uint32_t j0 = 0; j0 < n; j0 += 16) {
+        if (j0 + 16 < n) get(j0 + 16, vn);
+        mix16.template operator()<false>(pp[j0] * inv_lane, vr, j0, i);
+#pragma unroll
+        for (uint32_t j = 0; j < 16; ++j) vr[j] = vn[j];
+      }
+    }
+  }
+  // The outputs, and wo's input: each half-wave holds 32 dims of a pair, one Q8_0 block
+  // (quantize_block_lanes' steps, the four pairs side by side).
+  const size_t nbq = a.out_stride / kQK;
+  float d[4];
+#pragma unroll
+  for (uint32_t v = 0; v < 4; ++v) d[v] = half_wave_max(fabsf(acc[v])) / 127.0f;
+#pragma unroll
+  for (uint32_t v = 0; v < 4; ++v) {
+    const uint32_t pr = 4 * wave + v;
+    if (pvis[v] == 0) continue;
+    const uint32_t r = r0 + prow[v];
+    const size_t col = static_cast<size_t>(g * G + pr % G) * 64 + lane;
+    a.out[static_cast<size_t>(r) * a.out_stride + col] = acc[v];
+    if (a.outq != nullptr) {
+      const int32_t q = static_cast<int32_t>(roundf(acc[v] * (d[v] != 0.0f ? 1.0f / d[v] : 0.0f)));
+      const int32_t q_next = __builtin_amdgcn_update_dpp(0, q, 0xf5, 0xf, 0xf, true);  // quad_perm 1,1,3,3
+      uint8_t* block = a.outq + (static_cast<size_t>(r) * nbq + col / kQK) * kBytesQ8_0;
+      if ((lane & 31u) == 0) *reinterpret_cast<uint16_t*>(block) = static_cast<uint16_t>(float_to_half_bits(d[v]));
+      if ((lane & 1u) == 0)
+        *reinterpret_cast<uint16_t*>(block + 2 + (lane & 31u)) = static_cast<uint16_t>((q & 0xff) | ((q_next & 0xff) << 8));
+    }
+  }
+}
+
+// Dynamic LDS beyond 64 KB must be granted once per instantiation; false when the launch's LDS
+// exceeds what the device grants.
+template <bool F16, uint32_t G, uint32_t R>
+bool try_tile(const AttnArgs& a, uint32_t n_rows) {
+  static const size_t limit = [] {
+    int dev = 0, v = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
+      v = 65536;
+    v -= 512;  // the kernel's own exponential table
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(attention_tile_kernel<F16, G, R>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, v) != hipSuccess)
+      v = 65536 - 512;
+    return static_cast<size_t>(v);
+  }();
+  const size_t lds = tile_lds<F16, G, R>(a.max_vis);
+  if (lds > limit) return false;
+  hipLaunchKernelGGL((attention_tile_kernel<F16, G, R>), dim3((n_rows + R - 1) / R * a.n_kv), dim3(64 * tile_waves<G, R>()), lds,
+                     stream(), a, n_rows);
+  return true;
+}
+
+// Workgroups of 32 pairs where they leave one per CU and their scores fit; else of 16 where the
+// blocked kernel's do not (with both, the blocked kernel is the faster one: 128 rows behind 700
+// positions 58 against 66 us). Groups of 3 and 7 heads, whose waves would span rows, stay with the
+// blocked kernel (512 rows of 14 / 2 heads: 53 us either way).
+template <uint32_t G>
+bool launch_tile_g(const AttnArgs& a, uint32_t n_rows) {
+  auto attempt = [&]<uint32_t R>() {
+    if (static_cast<size_t>((n_rows + R - 1) / R) * a.n_kv < kTileMinWorkgroups) return false;
+    return a.f16 ? try_tile<true, G, R>(a, n_rows) : try_tile<false, G, R>(a, n_rows);
+  };
+  if (attempt.template operator()<32 / G>()) return true;
+  return block_lds(16, a.max_vis) > kBlockMaxLds && attempt.template operator()<16 / G>();
+}
+
+// The tiled kernel for whole-head launches of 64-dim heads and kv groups of 4 or 8 query heads;
+// false when it does not apply (the blocked or the one-row kernel runs instead).
+bool launch_tile(const AttnArgs& a, uint32_t n_rows) {
+  if (a.head_dim != 64 || a.head_begin != 0 || a.head_end != a.n_head) return false;
+  // A span's byte offsets are 32-bit.
+  if (static_cast<uint64_t>(a.max_vis) * a.n_kv * 64 * 4 >= (uint64_t(1) << 31)) return false;
+  switch (a.n_head / a.n_kv) {
+  case 4: return launch_tile_g<4>(a, n_rows);
+  case 8: return launch_tile_g<8>(a, n_rows);
   default: return false;
   }
 }
@@ -1667,6 +2133,9 @@ int attention_launch(const AttnArgs& a, uint32_t n_rows) {
     }
     return check_launch("attention (split)");
   }
+  // (Longer rows bring a scratch, which the tiled kernel leaves alone; without one they stay refused.
+  // 512 rows of 32 / 4 heads behind 1500 positions: 645 us in the one-row kernel, 500 here.)
+  if ((scores_fit_lds(a) || a.scratch != nullptr) && launch_tile(a, n_rows)) return check_launch("attention (tiled rows)");
   if (scores_fit_lds(a) && launch_block(a, n_rows)) return check_launch("attention (blocked rows)");
   if (a.outq != nullptr && a.head_dim % kQK != 0) {
     // The fused kernel quantizes whole 32-dim blocks only: quantize its output rows afterwards.

@@ -280,6 +280,69 @@ __device__ __forceinline__ int32_t dot32(const int32_t (&a)[8], const int32_t (&
   return s;
 }
 
+// ------------------------------------------------------------------------------------------
+// Reductions over lanes.
+
+template <int CTRL>
+__device__ __forceinline__ float max_dpp(float x) {
+  return fmaxf(x, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true)));
+}
+
+// The largest of a 16-lane row, in every lane of it: exchanges inside quads, halves and the row.
+__device__ __forceinline__ float row_max(float x) {
+  x = max_dpp<0xb1>(x);       // quad_perm 1,0,3,2
+  x = max_dpp<0x4e>(x);       // quad_perm 2,3,0,1
+  x = max_dpp<0x141>(x);      // row_half_mirror
+  return max_dpp<0x140>(x);   // row_mirror
+}
+
+// The largest of the 32 lanes of a half-wave: of its two rows, which meet by a swizzle (lane ^ 16).
+__device__ __forceinline__ float half_wave_max(float x) {
+  x = row_max(x);
+  return fmaxf(x, __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(x), 0x401f)));
+}
+
+// The largest of the 64 lanes, in every lane.
+__device__ __forceinline__ float wave_max(float x) {
+  x = row_max(x);
+  auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+}
+
+// x + the value of lane ^ 32, then lane ^ 16, lane ^ 8, ... lane ^ 1: the sum of the 64 lanes in
+// every lane, in the order of a descending __shfl_xor tree, without its LDS round trips (about 100
+// ns a step): halves and rows meet by lane swaps, rows of 16 by rotation (after the steps above, a
+// lane's value depends on its place in the half row only) and quads by permutation.
+template <int CTRL>
+__device__ __forceinline__ double dpp_double(double x) {
+  const uint64_t b = static_cast<uint64_t>(__double_as_longlong(x));
+  const uint32_t lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(b), CTRL, 0xf, 0xf, true);
+  const uint32_t hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(b >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double(static_cast<long long>((static_cast<uint64_t>(hi) << 32) | lo));
+}
+__device__ __forceinline__ double wave_sum(double x) {
+  uint64_t b = static_cast<uint64_t>(__double_as_longlong(x));
+  auto join = [](uint32_t lo, uint32_t hi) {
+    return __longlong_as_double(static_cast<long long>((static_cast<uint64_t>(hi) << 32) | lo));
+  };
+  uint32_t lo = static_cast<uint32_t>(b), hi = static_cast<uint32_t>(b >> 32);
+  auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+  auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+  x = join(l[0], h[0]) + join(l[1], h[1]);
+  b = static_cast<uint64_t>(__double_as_longlong(x));
+  lo = static_cast<uint32_t>(b);
+  hi = static_cast<uint32_t>(b >> 32);
+  l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+  h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+  x = join(l[0], h[0]) + join(l[1], h[1]);
+  x += dpp_double<0x128>(x);  // row_ror 8
+  x += dpp_double<0x124>(x);  // row_ror 4
+  x += dpp_double<0x4e>(x);   // quad_perm 2,3,0,1
+  return x + dpp_double<0xb1>(x);  // quad_perm 1,0,3,2
+}
+
 // Q8_0 quantization of one 32-element block held one element per lane in a 32-lane half-wave
 // (src/core/dtype.cpp:338-354): amax, d = amax / 127 (IEEE division), id = 1 / d or 0,
 // fp16(d), q = int8(roundf(x * id)), ties away from zero. `lane` is 0..31 within the half.

@@ -793,25 +793,6 @@ __device__ __forceinline__ float row_lane(float x) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x150 + L, 0xf, 0xf, true));  // row_newbcast
 }
 
-template <int CTRL>
-__device__ __forceinline__ float max_dpp(float x) {
-  return fmaxf(x, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true)));
-}
-
-// The largest of a 16-lane row, in every lane of it: exchanges inside quads, halves and the row.
-__device__ __forceinline__ float row_max(float x) {
-  x = max_dpp<0xb1>(x);       // quad_perm 1,0,3,2
-  x = max_dpp<0x4e>(x);       // quad_perm 2,3,0,1
-  x = max_dpp<0x141>(x);      // row_half_mirror
-  return max_dpp<0x140>(x);   // row_mirror
-}
-
-// The largest of the 32 lanes of a half-wave: of its two rows, which meet by a swizzle (lane ^ 16).
-__device__ __forceinline__ float half_wave_max(float x) {
-  x = row_max(x);
-  return fmaxf(x, __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(x), 0x401f)));
-}
-
 template <int T>
 __host__ __device__ constexpr uint32_t pair_dwords() { return (2 * block_bytes<T>() + 3) / 4; }
 

@@ -1,0 +1,106 @@
+"""Many-row attention with its products on the matrix cores (kv groups of 4 and 8 heads), where it
+can go wrong: rows that end inside a block, positions around the 64- and 32-position stages, the
+16-pair form of long contexts, spans that are not 16-byte aligned, blocks whose rows belong to
+different sequences, and values that are not finite past a row's own positions. Bit for bit against
+the oracle, the Q8_0 blocks of the outputs too."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from tables import CTable, HipTable
+
+pytestmark = pytest.mark.gpu
+HD = 64
+
+
+@pytest.fixture(scope="module")
+def o():
+    return CTable("oracle")
+
+
+@pytest.fixture(scope="module")
+def h():
+    return HipTable()
+
+
+def run(h, q, pool, k_off, v_off, n_vis, n_head, n_kv, f16):
+    H = h.H
+    n = len(n_vis)
+    bufs = [H.DeviceBuffer.of(a) for a in (q, pool, np.asarray(k_off, np.int64), np.asarray(v_off, np.int64),
+                                           np.asarray(n_vis, np.int32))]
+    out, outq = H.DeviceBuffer(n * n_head * HD * 4), H.DeviceBuffer(n * n_head * HD // 32 * 34)
+    a = H.AttentionRowsArgs()
+    a.q, a.kv, a.k_off, a.v_off, a.n_vis = (b.ptr for b in bufs)
+    a.out, a.outq, a.q_stride, a.out_stride = out.ptr, outq.ptr, n_head * HD, n_head * HD
+    a.n_head, a.n_kv, a.head_dim, a.scale, a.f16, a.max_vis = n_head, n_kv, HD, 0.125, int(f16), max(n_vis)
+    scratch = H.DeviceBuffer(4 * max(1, H.lib().axon_hip_attention_scratch_floats(C.byref(a), C.c_size_t(n))))
+    a.scratch = scratch.ptr
+    H.call("attention_rows", C.c_void_p(C.addressof(a)), n)
+    return out.download(np.float32).reshape(n, n_head, HD), outq.download(np.uint8)
+
+
+def check(o, h, chunk, past, decode, n_head, n_kv, f16, shift=0, poison=False, seed=1):
+    """A chunk of `chunk` rows behind `past` positions, then one row of each sequence in `decode`."""
+    rng = np.random.default_rng(seed)
+    seqs = [past + chunk] + list(decode)
+    n = chunk + len(decode)
+    row = n_kv * HD
+    q = rng.standard_normal((n, n_head, HD)).astype(np.float32)
+    kv = [(rng.standard_normal((m, row)).astype(np.float32), rng.standard_normal((m, row)).astype(np.float32)) for m in seqs]
+    if f16:
+        kv = [(k.astype(np.float16), v.astype(np.float16)) for k, v in kv]
+    want = np.zeros((n, n_head, HD), np.float32)
+    view = (lambda x: x.view(np.uint16)) if f16 else (lambda x: x)
+    want[:chunk] = o.attention_kv_heads(q[:chunk], view(kv[0][0]), view(kv[0][1]), chunk, past, n_head, n_kv, HD, 0.125,
+                                        0, n_head, f16=f16)
+    for i, m in enumerate(decode):
+        k, v = kv[1 + i]
+        want[chunk + i] = o.attention_kv_heads(q[chunk + i:chunk + i + 1], view(k), view(v), 1, m - 1, n_head, n_kv, HD,
+                                               0.125, 0, n_head, f16=f16)[0]
+    if poison:
+        # The last position is seen by the chunk's last row only: every other row's output must not
+        # take anything from it.
+        kv[0][0][-1] = np.nan
+        kv[0][1][-1] = np.inf
+    parts, k_off, v_off, at = [np.zeros(shift, kv[0][0].dtype)], [], [], shift
+    for k, v in kv:
+        k_off.append(at)
+        v_off.append(at + k.size)
+        parts += [k.ravel(), v.ravel()]
+        at += 2 * k.size
+    of = [0] * chunk + list(range(1, 1 + len(decode)))
+    n_vis = [past + i + 1 for i in range(chunk)] + list(decode)
+    got, blocks = run(h, q, np.concatenate(parts), [k_off[i] for i in of], [v_off[i] for i in of], n_vis, n_head, n_kv, f16)
+    keep = [r for r in range(n) if not (poison and r == chunk - 1)]
+    assert np.array_equal(got[keep].view(np.uint32), want[keep].view(np.uint32))
+    per_row = n_head * HD // 32 * 34
+    wq = h.quantize_row_q8_0(np.ascontiguousarray(want).ravel()).view(np.uint8).reshape(n, per_row)
+    assert np.array_equal(blocks.reshape(n, per_row)[keep], wq[keep])
+
+
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("chunk,past,n_head,n_kv", [
+    (250, 0, 32, 8),     # a last block of two rows; contexts from one position up
+    (257, 63, 32, 8),    # a last block of one row, contexts across the first K stage
+    (505, 31, 32, 4),    # groups of 8 heads: four rows per workgroup
+    (128, 1100, 32, 8),  # 16 pairs per workgroup
+    (128, 1030, 64, 8),  # the same with groups of 8
+])
+def test_chunk(o, h, chunk, past, n_head, n_kv, f16):
+    check(o, h, chunk, past, [], n_head, n_kv, f16)
+
+
+@pytest.mark.parametrize("f16", [False, True])
+def test_unaligned_span(o, h, f16):
+    check(o, h, 250, 20, [], 32, 8, f16, shift=1)
+
+
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("n_head,n_kv", [(32, 8), (64, 8)])
+def test_rows_of_other_sequences(o, h, n_head, n_kv, f16):
+    check(o, h, 243, 9, [1, 64, 65, 300, 17, 128, 33], n_head, n_kv, f16)
+
+
+def test_nothing_from_past_a_rows_positions(o, h):
+    check(o, h, 256, 15, [], 32, 8, False, poison=True)
