@@ -30,6 +30,7 @@
 #include <atomic>
 #include "common.h"
 #include "matvec.h"
+#include <type_traits>
 
 namespace axon_hip {
 
@@ -444,6 +445,145 @@ __global__ __launch_bounds__(TH) void q6k_planar_kernel(MatvecArgs args, uint32_
   }
 }
 
+// Many activation rows over the planar copy, the products on the matrix cores. A lane still owns an
+// output row and decodes its super-blocks, but its value meets S = 32 or 16 activation rows in one
+// f32 outer product with a zero addend (v_mfma_f32_32x32x1: two blocks of 32 output rows; 16x16x1:
+// four of 16), each element rounded once as the product is (a zero product comes out +0, which no
+// sum that starts at +0 can tell); the vector ALU only adds, element after element. What
+// bounded q6k_planar_kernel here was the multiply's scalar operand: v_mul_f32 with one issues at
+// half rate, 1.72 ns a SIMD against 0.97 for an add, where the outer product is 0.84 an element and
+// takes its activations from registers that one 16-byte load per lane fills for 8 (or 16) steps.
+// Measured at 128256 x 2048, us: 32 rows 427 -> 303, 16 rows 242 -> 178, 64 rows 843 -> 591.
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x32 __attribute__((ext_vector_type(32)));
+
+// Half a super-block of one row: elements 128 n .. 128 n + 127.
+struct PlanarHalf {
+  u32x4 ql[4], qh[2];
+  u32x4 sc;    // all 16 scales
+  uint32_t d;
+};
+
+__device__ __forceinline__ void planar_fetch_half(const uint8_t* col, uint32_t n_out, uint32_t row, uint32_t n,
+                                                  PlanarHalf& b) {
+  auto slice = [&](uint32_t s) {
+    return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(col + static_cast<size_t>(s) * 16 * n_out) + row);
+  };
+#pragma unroll
+  for (uint32_t i = 0; i < 4; ++i) b.ql[i] = slice(4 * n + i);
+#pragma unroll
+  for (uint32_t i = 0; i < 2; ++i) b.qh[i] = slice(8 + 2 * n + i);
+  b.sc = slice(12);
+  b.d = reinterpret_cast<const uint16_t*>(col + static_cast<size_t>(208) * n_out)[row];
+}
+
+template <int I, int N, typename F>
+__device__ __forceinline__ void for_each_index(F f) {
+  if constexpr (I < N) {
+    f.template operator()<I>();
+    for_each_index<I + 1, N>(f);
+  }
+}
+
+template <uint32_t S>
+__global__ __launch_bounds__(256, 2) void q6k_planar_mfma_kernel(MatvecArgs args, uint32_t n_in, size_t col_bytes,
+                                                                 uint32_t m_total) {
+  static_assert(S == 32 || S == 16, "32 or 16 activation rows");
+  constexpr uint32_t kGroups = 64 / S;     // output-row blocks of one outer product, and x groups per load
+  constexpr uint32_t kPer = 4 * kGroups;   // elements that one load per lane covers
+  constexpr uint32_t ND = S * S * kGroups / 64;  // products per lane
+  typedef std::conditional_t<S == 32, f32x32, f32x16> Products;
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
+  const MatvecSeg seg = args.seg[0];
+  const uint32_t m0 = blockIdx.x * S;
+  const uint32_t mm = min(S, m_total - m0);
+  const uint32_t row_id = blockIdx.y * 256 + tid;
+  const uint32_t row = min(row_id, seg.n_out - 1);  // past the last row: read it, store nothing
+  // Lane l holds elements kPer t + 4 (l / S) .. + 3 of activation row l % S (rows past the last read it).
+  const float4* x = reinterpret_cast<const float4*>(reinterpret_cast<const float*>(args.xq) +
+                                                    static_cast<size_t>(m0 + min(lane % S, mm - 1)) * n_in + 4 * (lane / S));
+  constexpr uint32_t kStep = kPer / 4;  // float4 between loads
+  const uint32_t n_loads = n_in / kPer;
+  float acc[ND];
+#pragma unroll
+  for (uint32_t v = 0; v < ND; ++v) acc[v] = 0.0f;
+  constexpr uint32_t kLoads = 128 / kPer;  // x loads per half
+  constexpr uint32_t kAhead = 4;           // x loads in flight
+  static_assert(kLoads % kAhead == 0, "the ring's slots are static");
+  float4 xr[kAhead];
+#pragma unroll
+  for (uint32_t t = 0; t < kAhead; ++t) xr[t] = x[t * kStep];
+
+  const uint32_t halves = 2 * args.nb;
+  PlanarHalf cur, next;
+  planar_fetch_half(seg.w, seg.n_out, row, 0, cur);
+  for (uint32_t u = 0; u < halves; ++u) {
+    const uint32_t w = min(u + 1, halves - 1);
+    planar_fetch_half(seg.w + static_cast<size_t>(w >> 1) * col_bytes, seg.n_out, row, w & 1, next);
+    const float d = half_value(cur.d);
+    const uint32_t sc[2] = {(u & 1) != 0 ? cur.sc[2] : cur.sc[0], (u & 1) != 0 ? cur.sc[3] : cur.sc[1]};
+    // The value of element 4 st + e of the half: (d * scale) * (q - 32), as planar_superblock forms it.
+    float val[4];
+    auto decode = [&](int st) {
+      const int qi = (st / 8) % 4, hf = (st / 4) % 2, l4 = st % 4;
+      const int si = qi * 2 + hf;
+      const float scale = static_cast<float>(static_cast<int8_t>((sc[si >> 2] >> (8 * (si & 3))) & 0xffu));
+      const float ds = d * scale;       // exact
+      const float neg32 = -32.0f * ds;  // exact
+      const int l = 16 * hf + 4 * l4;
+      const int lo = 32 * (qi & 1) + l;
+      const uint32_t lw = cur.ql[lo / 16][(lo / 4) & 3];
+      const uint32_t hw = cur.qh[l / 16][(l / 4) & 3];
+      const uint32_t q = ((lw >> (4 * (qi >> 1))) & 0x0f0f0f0fu) | (((hw >> (2 * qi)) & 0x03030303u) << 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) val[e] = fmaf(ds, static_cast<float>((q >> (8 * e)) & 0xffu), neg32);
+    };
+    Products p[2];
+    auto outer = [&]<int ST, int E>(Products& out) {
+      const float4 xv = xr[ST / kGroups % kAhead];
+      const float xe = E == 0 ? xv.x : E == 1 ? xv.y : E == 2 ? xv.z : xv.w;
+      constexpr int kGroup = ST % kGroups;
+      const Products zero = {};
+      if constexpr (S == 32) out = __builtin_amdgcn_mfma_f32_32x32x1f32(xe, val[E], zero, 1, kGroup, 0);
+      else out = __builtin_amdgcn_mfma_f32_16x16x1f32(xe, val[E], zero, 2, kGroup, 0);
+    };
+    auto add = [&](const Products& in) {
+#pragma unroll
+      for (uint32_t v = 0; v < ND; ++v) acc[v] += in[v];
+    };
+    decode(0);
+    outer.template operator()<0, 0>(p[0]);
+    for_each_index<0, 128>([&]<int K>() {
+      // Element K's products are in p[K % 2]; element K + 1's are formed while they are added.
+      constexpr int N = K + 1;
+      if constexpr (N < 128) {
+        if constexpr (N % 4 == 0) decode(N / 4);
+        outer.template operator()<N / 4, N % 4>(p[N % 2]);
+        if constexpr (N % kPer == kPer - 1) {
+          // The last element of an x load has been taken: its slot takes the load kAhead further.
+          const uint32_t t = u * kLoads + N / kPer + kAhead;
+          xr[N / kPer % kAhead] = x[min(t, n_loads - 1) * kStep];
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      add(p[K % 2]);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    cur = next;
+  }
+  // Lane l, product v: output row (v / (ND / kGroups)) * S + l % S of the wave's 64, activation row
+  // 8 (v' / 4) + 4 (l / 32) + v' % 4 (S = 32) or 4 (l / 16) + v' (S = 16) for v' = v % (ND / kGroups).
+  constexpr uint32_t kV = ND / kGroups;
+  const uint32_t wave_row = row_id - lane;
+#pragma unroll
+  for (uint32_t v = 0; v < ND; ++v) {
+    const uint32_t o = wave_row + v / kV * S + lane % S;
+    const uint32_t vv = v % kV;
+    const uint32_t m = S == 32 ? 8 * (vv / 4) + 4 * (lane / 32) + vv % 4 : 4 * (lane / 16) + vv;
+    if (o < seg.n_out && m < mm) seg.y[static_cast<size_t>(m0 + m) * seg.y_stride + o] = acc[v];
+  }
+}
+
 // One activation row against a short matrix: R output rows per workgroup, the products apart
 // from the sums. The threads take units of (super-block, quarter, row) and write the quarter's
 // 64 products v * x in element order into LDS ([super-block][row][256 + 4 pad] floats); then lane
@@ -854,6 +994,33 @@ int matvec_q6k_planar_launch(MatvecArgs& a, uint32_t n_in) {
       default: ok = chain_granted<1>(chain_lds<1>(nsb)); if (ok) launch(q6k_planar_chain_kernel<1>, dim3(blocks), dim3(256), chain_lds<1>(nsb), a, n_in, col_bytes); break;
     }
     if (ok) return check_launch("q6k_planar_chain");
+  }
+  // Whole chunks of activation rows on the matrix cores where they give the chip its waves of 64
+  // output rows (two per SIMD for 32-row chunks, one for 16-row ones); the rows left over, and short
+  // matrices, on the vector ALU below. 128256 x 2048, us: 9 rows 170 there against 177 in one 16-row
+  // chunk, 12 rows 188 / 177, 16 + 4 rows 316 / 258, 24 rows 328 / 299 in one 32-row chunk; 64000 rows
+  // (1000 waves) at 16 rows 128 / 110, 32000 rows at 16 rows 79 / 110 and at 32 rows 127 / 112.
+  {
+    const uint32_t waves = static_cast<uint32_t>(ceil_div(n_out, 64));
+    const uint32_t blocks = static_cast<uint32_t>(ceil_div(n_out, 256));
+    const float* x = reinterpret_cast<const float*>(a.xq);
+    MatvecArgs g = a;
+    auto take = [&](auto kernel, uint32_t chunks, uint32_t rows) {
+      g.m = std::min(a.m, chunks * rows);
+      launch(kernel, dim3(chunks, blocks), dim3(256), 0, g, n_in, col_bytes, g.m);
+      a.m -= g.m;
+      x += static_cast<size_t>(g.m) * n_in;
+      a.xq = reinterpret_cast<const uint8_t*>(x);
+      a.seg[0].y += static_cast<size_t>(g.m) * a.seg[0].y_stride;
+      g = a;
+    };
+    const uint32_t c32 = a.m / 32 + (a.m % 32 >= 23 ? 1 : 0);
+    if (blocks <= 65535 && static_cast<uint64_t>(c32) * waves >= 1536) take(q6k_planar_mfma_kernel<32>, c32, 32);
+    const uint32_t c16 = a.m / 16 + (a.m % 16 >= 10 ? 1 : 0);
+    // (With one wave per SIMD only where no rows are left over: 64000 rows at 24, 177 / 185 us.)
+    if (blocks <= 65535 && static_cast<uint64_t>(c16) * waves >= (c16 * 16 >= a.m ? 896 : 1536))
+      take(q6k_planar_mfma_kernel<16>, c16, 16);
+    if (a.m == 0) return check_launch("q6k_planar_mfma");
   }
   // Activation rows per workgroup: up to kQ6MaxRows (each lane then runs that many chains, and
   // every weight slice is read once per that many rows), but fewer while that leaves under 1024

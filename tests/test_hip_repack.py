@@ -283,3 +283,36 @@ def test_model_logits_unchanged_by_the_repack(H, tmp_path_factory):
         m.close()
     assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
     assert out[0][2] - out[1][2] == 2048 * 2048 // 256 * 210
+
+
+@pytest.mark.parametrize("n_rows,n_out,n_in", [
+    (10, 57409, 256),   # one 16-row chunk with 6 rows missing; the last wave holds one output row
+    (16, 98305, 512),   # a whole 16-row chunk
+    (19, 98400, 256),   # 16 rows and 3 on the vector ALU
+    (32, 98305, 256),   # a whole 32-row chunk
+    (55, 98310, 512),   # two 32-row chunks, 9 rows missing
+    (70, 98310, 256),   # two 32-row chunks and 6 rows
+])
+def test_planar_many_rows(H, o, n_rows, n_out, n_in):
+    """The matrix-core kernels' chunks and left-over rows, with strided outputs: the same rows in
+    calls of at most 8 (the vector-ALU kernel), and the oracle for the first and the last row."""
+    w = q6k_weights(n_out, n_in, 21)
+    w["d"][5] = 0xfc00  # an infinite and a NaN scale stay in their rows
+    w["d"][-1] = 0x7e00
+    planar, _ = repack(H, w, n_out, n_in)
+    x = random_floats(n_rows * n_in, 22, 2.0).reshape(n_rows, n_in)
+    x[0, 3] = -0.0
+    x[n_rows - 1, 7] = np.inf
+    dx = H.DeviceBuffer.of(x)
+    stride = n_out + 3
+    y = H.DeviceBuffer.of(np.full(n_rows * stride, np.float32(-7.25), np.float32))
+    H.call("matmul_q6_k_planar", planar, dx, y, n_rows, n_out, n_in, stride)
+    got = y.download(np.float32).reshape(n_rows, stride)
+    assert np.all(got[:, n_out:] == np.float32(-7.25))
+    for r0 in range(0, n_rows, 8):
+        m = min(8, n_rows - r0)
+        part = H.DeviceBuffer(m * n_out * 4)
+        H.call("matmul_q6_k_planar", planar, dx.at(r0 * n_in * 4), part, m, n_out, n_in, n_out)
+        assert np.array_equal(got[r0:r0 + m, :n_out], part.download(np.float32).reshape(m, n_out), equal_nan=True)
+    for r in (0, n_rows - 1):
+        assert np.array_equal(got[r, :n_out], o.matmul("q6_k", w, x[r], n_out, n_in), equal_nan=True)
