@@ -1,0 +1,51 @@
+"""F32 / F16 / BF16 weights against float activations around the kernel's tiles (16 outputs x 16 rows,
+chunks of 256 elements, two loaded ahead): odd sizes, one to three chunks and more, strided outputs,
+special values; bit for bit against the oracle."""
+import numpy as np
+import pytest
+
+from tables import CTable, HipTable, random_floats
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def o():
+    return CTable("oracle")
+
+
+@pytest.fixture(scope="module")
+def h():
+    return HipTable()
+
+
+def weights(kind, n, seed):
+    w = random_floats(n, seed, 2.0)
+    w[::97] = -0.0
+    w[5::501] = 1e-7  # below the smallest normal half
+    if kind == "f16":
+        return w.astype(np.float16).view(np.uint16)
+    return (w.view(np.uint32) >> 16).astype(np.uint16) if kind == "bf16" else w
+
+
+@pytest.mark.parametrize("kind", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("n_rows,n_out,n_in", [(1, 1, 1), (1, 17, 255), (3, 16, 256), (16, 33, 257), (17, 15, 513),
+                                               (33, 50, 1031), (2, 300, 2048)])
+def test_float_matmul_tiles(o, h, kind, n_rows, n_out, n_in):
+    w, x = weights(kind, n_out * n_in, 1), random_floats(n_rows * n_in, 2, 3.0)
+    stride = n_out + 2
+    want = o.matmul(kind, w, x, n_out, n_in, n_rows=n_rows, y_stride=stride)
+    got = h.matmul(kind, w, x, n_out, n_in, n_rows=n_rows, y_stride=stride)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    if n_rows == 1:
+        assert np.array_equal(h.matmul(kind, w, x, n_out, n_in).view(np.uint32), want[:n_out].view(np.uint32))
+
+
+@pytest.mark.parametrize("kind", ["f32", "f16", "bf16"])
+def test_float_matmul_infinities_stay_in_their_row(o, h, kind):
+    n_rows, n_out, n_in = 18, 20, 300
+    w, x = weights(kind, n_out * n_in, 3), random_floats(n_rows * n_in, 4)
+    x[7 * n_in + 299] = np.inf
+    x[17 * n_in] = np.nan
+    want = o.matmul(kind, w, x, n_out, n_in, n_rows=n_rows)
+    assert np.array_equal(h.matmul(kind, w, x, n_out, n_in, n_rows=n_rows), want, equal_nan=True)
