@@ -287,6 +287,51 @@ def test_topk_rows_match_sorted_order(H, n, k):
         assert np.array_equal(got_v[r].view(np.uint32), want_v.view(np.uint32)), kind
 
 
+@pytest.mark.parametrize("n", [256, 1023, 1025, 20000])
+@pytest.mark.parametrize("k", [1, 255, 256])
+def test_topk_rows_threshold_edges(H, n, k):
+    """Rows at the edges of the threshold that gathers the candidates: k - 1, k and 1023 to 1025
+    finite values over -inf, as many values above a tied floor, infinities, a NaN row, values
+    around zero and denormals, and values that agree in all but their last bits."""
+    rng = np.random.default_rng(7 * n + k)
+    rows = []
+    for low in (-np.inf, np.nan, -1.0, np.finfo(np.float32).min):
+        for count in (0, k - 1, k, 1023, 1024, 1025):
+            x = np.full(n, low, np.float32)
+            at = rng.permutation(n)[:min(count, n)]
+            x[at] = rng.standard_normal(len(at)).astype(np.float32)
+            rows.append(x)
+    bits = rng.integers(0, 2048, n).astype(np.uint32)
+    rows.append((bits | 0x3f800000).astype(np.uint32).view(np.float32))   # one bound for all
+    rows.append((bits | 0xbf800000).astype(np.uint32).view(np.float32))
+    rows.append(bits.view(np.float32))                                   # denormals, zeros
+    rows.append((bits | 0x80000000).astype(np.uint32).view(np.float32))
+    x = rng.standard_normal(n).astype(np.float32)
+    x[rng.integers(0, n, 20)] = np.inf
+    x[rng.integers(0, n, 20)] = -np.inf
+    rows.append(x)
+    for high in (40, 300):            # many equal values, few above them, the rest below
+        x = np.full(n, -2.0, np.float32)
+        at = rng.permutation(n)
+        x[at[:n // 2]] = 1.5
+        x[at[:min(high, n)]] = rng.random(min(high, n)).astype(np.float32) + 2
+        rows.append(x)
+    x = rng.standard_normal(n).astype(np.float32)
+    x[np.arange(n) % 1024 < 90] += 50  # more than 1024 large values, all with few threads
+    rows.append(x)
+    x = np.stack(rows)
+    dx = H.DeviceBuffer.of(x)
+    ol = H.DeviceBuffer(4 * len(x) * k)
+    oi = H.DeviceBuffer(4 * len(x) * k)
+    H.call("topk_rows", dx, n, len(x), n, k, ol, oi)
+    got_v = ol.download(np.float32, len(x) * k).reshape(len(x), k)
+    got_i = oi.download(np.int32, len(x) * k).reshape(len(x), k)
+    for r in range(len(x)):
+        want_v, want_i = topk_reference(x[r], k)
+        assert np.array_equal(got_i[r], want_i), r
+        assert np.array_equal(got_v[r].view(np.uint32), want_v.view(np.uint32)), r
+
+
 def test_topk_rows_bounds(H):
     dx = H.DeviceBuffer.of(np.zeros(300, np.float32))
     out = H.DeviceBuffer(4 * 300)
