@@ -1,6 +1,7 @@
-"""F32 / F16 / BF16 weights against float activations around the kernel's tiles (16 outputs x 16 rows,
-chunks of 256 elements, two loaded ahead): odd sizes, one to three chunks and more, strided outputs,
-special values; bit for bit against the oracle."""
+"""F32 / F16 / BF16 weights against float activations around the kernel's tiles (16 outputs x 16 or 32
+rows, chunks of 256 elements, two loaded ahead): odd sizes, one to three chunks and more, strided
+outputs, weights that pairs of elements are not aligned for, special values; bit for bit against the
+oracle."""
 import numpy as np
 import pytest
 
@@ -49,3 +50,26 @@ def test_float_matmul_infinities_stay_in_their_row(o, h, kind):
     x[17 * n_in] = np.nan
     want = o.matmul(kind, w, x, n_out, n_in, n_rows=n_rows)
     assert np.array_equal(h.matmul(kind, w, x, n_out, n_in, n_rows=n_rows), want, equal_nan=True)
+
+
+# Both row counts of a tile on whole and partial ones: 32 rows up to 16 rows of input, and from 256
+# workgroups on; 16 rows between.
+@pytest.mark.parametrize("kind", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("n_rows,n_out,n_in", [(16, 32, 512), (17, 32, 768), (31, 4100, 270), (33, 2049, 512), (65, 1366, 258)])
+def test_float_matmul_tile_heights(o, h, kind, n_rows, n_out, n_in):
+    w, x = weights(kind, n_out * n_in, 5), random_floats(n_rows * n_in, 6, 3.0)
+    want = o.matmul(kind, w, x, n_out, n_in, n_rows=n_rows)
+    got = h.matmul(kind, w, x, n_out, n_in, n_rows=n_rows)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("kind", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("n_rows", [3, 20])
+def test_float_matmul_weights_off_pair_alignment(o, h, kind, n_rows):
+    """Even rows from an address that is a whole element, not a whole pair; activations off 16 bytes."""
+    n_out, n_in = 35, 514
+    w, x = weights(kind, n_out * n_in + 1, 7), random_floats(n_rows * n_in + 1, 8, 3.0)
+    dw, dx, y = h._dev(w), h._dev(x), h._dev(np.zeros(n_rows * n_out, np.float32))
+    h.H.call(f"matmul_{kind}_rows", dw.at(w.itemsize), dx.at(4), y, n_rows, n_out, n_in, n_out)
+    want = o.matmul(kind, w[1:].copy(), x[1:].copy(), n_out, n_in, n_rows=n_rows)
+    assert np.array_equal(y.download(np.float32).view(np.uint32), want.view(np.uint32))
