@@ -33,7 +33,7 @@ constexpr uint32_t kVMaxItems = kVTile * 128 / 4 / kThreads;  // 4-float items p
 constexpr uint32_t kBlockMinWorkgroups = 512;
 constexpr size_t kBlockMaxLds = 80 * 1024;
 constexpr int kBlockWaves = 3;  // waves per SIMD the blocked kernel's registers allow
-// The tiled many-row kernel: only while its blocks leave a workgroup per CU.
+// The tiled many-row kernel: only while its blocks leave a workgroup per CU (two of the smaller ones).
 constexpr uint32_t kTileMinWorkgroups = 256;
 
 __host__ __device__ inline uint32_t round4(uint32_t v) { return (v + 3) & ~3u; }
@@ -1156,12 +1156,15 @@ bool try_tile(const AttnArgs& a, uint32_t n_rows) {
 
 // Workgroups of 32 pairs where they leave one per CU and their scores fit; else of 16 where the
 // blocked kernel's do not (with both, the blocked kernel is the faster one: 128 rows behind 700
-// positions 58 against 66 us). Groups of 3 and 7 heads, whose waves would span rows, stay with the
+// positions 58 against 66 us) and two workgroups per CU are there: its single rows spread wider below
+// that (32 / 4 heads: 163 rows behind 885 positions, 328 workgroups, 88 against 135 us, 195 behind
+// 1001, 392 workgroups, 139 against 155). Groups of 3 and 7 heads, whose waves would span rows, stay with the
 // blocked kernel (512 rows of 14 / 2 heads: 53 us either way).
 template <uint32_t G>
 bool launch_tile_g(const AttnArgs& a, uint32_t n_rows) {
   auto attempt = [&]<uint32_t R>() {
-    if (static_cast<size_t>((n_rows + R - 1) / R) * a.n_kv < kTileMinWorkgroups) return false;
+    constexpr size_t kLeast = G * R == 32 ? kTileMinWorkgroups : 2 * kTileMinWorkgroups;
+    if (static_cast<size_t>((n_rows + R - 1) / R) * a.n_kv < kLeast) return false;
     return a.f16 ? try_tile<true, G, R>(a, n_rows) : try_tile<false, G, R>(a, n_rows);
   };
   if (attempt.template operator()<32 / G>()) return true;

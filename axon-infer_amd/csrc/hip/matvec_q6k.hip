@@ -998,7 +998,7 @@ int matvec_q6k_planar_launch(MatvecArgs& a, uint32_t n_in) {
   // Whole chunks of activation rows on the matrix cores where they give the chip its waves of 64
   // output rows (two per SIMD for 32-row chunks, one for 16-row ones); the rows left over, and short
   // matrices, on the vector ALU below. 128256 x 2048, us: 9 rows 170 there against 177 in one 16-row
-  // chunk, 12 rows 188 / 177, 16 + 4 rows 316 / 258, 24 rows 328 / 299 in one 32-row chunk; 64000 rows
+  // chunk, 12 rows 188 / 177, 16 + 4 rows 316 / 258, 24 rows 328 / 299 in one 32-row chunk (106305 x 1536 at 23: 223 / 231); 64000 rows
   // (1000 waves) at 16 rows 128 / 110, 32000 rows at 16 rows 79 / 110 and at 32 rows 127 / 112.
   {
     const uint32_t waves = static_cast<uint32_t>(ceil_div(n_out, 64));
@@ -1014,7 +1014,7 @@ int matvec_q6k_planar_launch(MatvecArgs& a, uint32_t n_in) {
       a.seg[0].y += static_cast<size_t>(g.m) * a.seg[0].y_stride;
       g = a;
     };
-    const uint32_t c32 = a.m / 32 + (a.m % 32 >= 23 ? 1 : 0);
+    const uint32_t c32 = a.m / 32 + (a.m % 32 >= 24 ? 1 : 0);
     if (blocks <= 65535 && static_cast<uint64_t>(c32) * waves >= 1536) take(q6k_planar_mfma_kernel<32>, c32, 32);
     const uint32_t c16 = a.m / 16 + (a.m % 16 >= 10 ? 1 : 0);
     // (With one wave per SIMD only where no rows are left over: 64000 rows at 24, 177 / 185 us.)

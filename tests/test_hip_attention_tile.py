@@ -84,8 +84,10 @@ def check(o, h, chunk, past, decode, n_head, n_kv, f16, shift=0, poison=False, s
     (250, 0, 32, 8),     # a last block of two rows; contexts from one position up
     (257, 63, 32, 8),    # a last block of one row, contexts across the first K stage
     (505, 31, 32, 4),    # groups of 8 heads: four rows per workgroup
-    (128, 1100, 32, 8),  # 16 pairs per workgroup
+    (128, 1100, 32, 8),  # 16 pairs' LDS, too few workgroups for them
     (128, 1030, 64, 8),  # the same with groups of 8
+    (64, 1100, 128, 32),  # both again at the 512 workgroups that 16 pairs ask for
+    (64, 1030, 128, 16),
 ])
 def test_chunk(o, h, chunk, past, n_head, n_kv, f16):
     check(o, h, chunk, past, [], n_head, n_kv, f16)
