@@ -1,8 +1,10 @@
 /*
  * TEST INFRASTRUCTURE ONLY (the CPU oracle; see oracle.h). The forward pass restated from
- * src/model/llama.cpp:315-639 and the sampler from src/sampling/sampler.cpp:66-183. Single
- * threaded: the reference splits columns and heads across threads so that no reduction ever
- * crosses a thread (llama.cpp:310-314), which makes one thread give the same bits.
+ * src/model/llama.cpp:315-639 and the sampler from src/sampling/sampler.cpp:66-183. Columns of a
+ * matmul and (row, head) pairs of the attention are split across threads, as in the reference
+ * (llama.cpp:310-314): no reduction ever crosses a thread, so any number of threads gives the
+ * same bits (tests/test_oracle_threads.py). One thread takes over a minute for a 512-row pass of a
+ * 1B-parameter model.
  */
 #include "oracle.h"
 
@@ -62,37 +64,45 @@ static size_t row_bytes(const ora_tensor* w) {
   }
 }
 
-/* llama.cpp:30-101 matmul_columns over every column: rows are independent, and the _rows
+/* Columns o0 .. o0 + n - 1 of llama.cpp:30-101 matmul_columns: rows are independent, and the _rows
  * entries are the single-row entries looped (ref/quant.cpp:111-139), so one row at a time. */
-static void matmul(const ora_model* m, const ora_tensor* w, const float* x, const ora_block_q8_0* xq,
-                   float* y, size_t n_rows, size_t y_stride) {
-  const size_t n_in = w->ne0, n_out = w->ne1, nb = n_in / 32;
+static void matmul_columns(const ora_model* m, const ora_tensor* w, const float* x, const ora_block_q8_0* xq,
+                           float* y, size_t n_rows, size_t y_stride, size_t o0, size_t n) {
+  const size_t n_in = w->ne0, nb = n_in / 32;
+  const void* data = (const char*)w->data + o0 * row_bytes(w);
   const int exact = m->exact_activations;
-  (void)row_bytes;
   for (size_t r = 0; r < n_rows; ++r) {
     const float* xr = x + r * n_in;
     const ora_block_q8_0* xqr = xq != NULL ? xq + r * nb : NULL;
-    float* yr = y + r * y_stride;
+    float* yr = y + r * y_stride + o0;
     switch (w->type) {
-    case ORA_F32: ora_matmul_f32(w->data, xr, yr, n_out, n_in); break;
-    case ORA_F16: ora_matmul_f16(w->data, xr, yr, n_out, n_in); break;
-    case ORA_BF16: ora_matmul_bf16(w->data, xr, yr, n_out, n_in); break;
+    case ORA_F32: ora_matmul_f32(data, xr, yr, n, n_in); break;
+    case ORA_F16: ora_matmul_f16(data, xr, yr, n, n_in); break;
+    case ORA_BF16: ora_matmul_bf16(data, xr, yr, n, n_in); break;
     case ORA_Q8_0:
-      if (exact) ora_matmul_q8_0(w->data, xr, yr, n_out, n_in);
-      else ora_matmul_q8_0_q8(w->data, xqr, yr, n_out, n_in);
+      if (exact) ora_matmul_q8_0(data, xr, yr, n, n_in);
+      else ora_matmul_q8_0_q8(data, xqr, yr, n, n_in);
       break;
     case ORA_Q4_0:
-      if (exact) ora_matmul_q4_0(w->data, xr, yr, n_out, n_in);
-      else ora_matmul_q4_0_q8(w->data, xqr, yr, n_out, n_in);
+      if (exact) ora_matmul_q4_0(data, xr, yr, n, n_in);
+      else ora_matmul_q4_0_q8(data, xqr, yr, n, n_in);
       break;
     case ORA_Q4_1:
-      if (exact) ora_matmul_q4_1(w->data, xr, yr, n_out, n_in);
-      else ora_matmul_q4_1_q8(w->data, xqr, yr, n_out, n_in);
+      if (exact) ora_matmul_q4_1(data, xr, yr, n, n_in);
+      else ora_matmul_q4_1_q8(data, xqr, yr, n, n_in);
       break;
-    case ORA_Q6_K: ora_matmul_q6_k(w->data, xr, yr, n_out, n_in); break;
+    case ORA_Q6_K: ora_matmul_q6_k(data, xr, yr, n, n_in); break;
     default: break;
     }
   }
+}
+
+static void matmul(const ora_model* m, const ora_tensor* w, const float* x, const ora_block_q8_0* xq,
+                   float* y, size_t n_rows, size_t y_stride) {
+  enum { kColumns = 32 }; /* columns per item: a weight row is read once for all activation rows */
+#pragma omp parallel for schedule(dynamic)
+  for (size_t o = 0; o < w->ne1; o += kColumns)
+    matmul_columns(m, w, x, xq, y, n_rows, y_stride, o, w->ne1 - o < kColumns ? w->ne1 - o : kColumns);
 }
 
 /* llama.cpp:401-417: the input is quantized once per launch that feeds quantized weights. */
@@ -153,6 +163,33 @@ static uint16_t* cache_v16(const ora_model* m, ora_cache* c, size_t l) {
 /* llama.cpp:525-532, 559-563: rows of float keys and values rounded once into an fp16 cache. */
 static void round_in(uint16_t* dst, const float* src, size_t n) {
   for (size_t i = 0; i < n; ++i) dst[i] = ora_fp32_to_fp16(src[i]);
+}
+
+/* Every row's heads, llama.cpp:520-556 (a batch: row i over batch[i]'s cache at its position) and
+ * 566-590 (a chunk: row i over k, v at n_past + i). Each row is a call of its own, as its scores are its
+ * own row of the workspace. */
+static void attend(const ora_model* m, const float* q, ora_cache* const* batch, size_t l, const void* k,
+                   const void* v, float* out, float* scores, size_t seq, size_t total, size_t n_past, int half,
+                   float scale) {
+  const size_t nh = m->n_head, nkv = m->n_head_kv, hd = m->head_dim, q_row = nh * hd;
+#pragma omp parallel for schedule(dynamic)
+  for (size_t i = 0; i < seq; ++i) {
+    const size_t past = batch != NULL ? batch[i]->pos : n_past + i;
+    const void* ki = k;
+    const void* vi = v;
+    if (batch != NULL && half) {
+      ki = cache_k16(m, batch[i], l);
+      vi = cache_v16(m, batch[i], l);
+    } else if (batch != NULL) {
+      ki = cache_k(m, batch[i], l);
+      vi = cache_v(m, batch[i], l);
+    }
+    const float* qi = q + i * q_row;
+    float* oi = out + i * q_row;
+    float* si = scores + i * total; /* past + 1 <= total */
+    if (half) ora_attention_kv_heads_f16(qi, ki, vi, oi, si, 1, past, nh, nkv, hd, scale, 0, nh);
+    else ora_attention_kv_heads(qi, ki, vi, oi, si, 1, past, nh, nkv, hd, scale, 0, nh);
+  }
 }
 
 /* The one forward pass, llama.cpp:315-639. batch != NULL is forward_batch: row i is its own
@@ -223,32 +260,16 @@ static int run(const ora_model* m, const int32_t* tokens, size_t seq, ora_cache*
           memcpy(cache_v(m, c, l) + c->pos * kv_row, v_new + i * kv_row, kv_row * sizeof(float));
         }
       }
-      for (size_t b = 0; b < seq; ++b) {
-        ora_cache* c = batch[b];
-        for (size_t h = 0; h < nh; ++h) {
-          if (half_cache)
-            ora_attention_kv_heads_f16(a.q + b * q_row, cache_k16(m, c, l), cache_v16(m, c, l),
-                                       a.attn + b * q_row, a.scores, 1, c->pos, nh, nkv, hd, scale, h, h + 1);
-          else
-            ora_attention_kv_heads(a.q + b * q_row, cache_k(m, c, l), cache_v(m, c, l), a.attn + b * q_row,
-                                   a.scores, 1, c->pos, nh, nkv, hd, scale, h, h + 1);
-        }
-      }
+      attend(m, a.q, batch, l, NULL, NULL, a.attn, a.scores, seq, total, 0, half_cache, scale);
     } else if (half_cache) {
       /* llama.cpp:557-563 then 566-590: the chunk's rows rounded in, then every row attends over
        * the fp16 cache. */
       round_in(cache_k16(m, cache, l) + n_past * kv_row, k_new, seq * kv_row);
       round_in(cache_v16(m, cache, l) + n_past * kv_row, v_new, seq * kv_row);
-      for (size_t h = 0; h < nh; ++h) {
-        ora_attention_kv_heads_f16(a.q, cache_k16(m, cache, l), cache_v16(m, cache, l), a.attn, a.scores, seq,
-                                   n_past, nh, nkv, hd, scale, h, h + 1);
-      }
+      attend(m, a.q, NULL, l, cache_k16(m, cache, l), cache_v16(m, cache, l), a.attn, a.scores, seq, total, n_past, 1,
+             scale);
     } else {
-      /* llama.cpp:566-590: rows are computed independently, so all rows in one call. */
-      for (size_t h = 0; h < nh; ++h) {
-        ora_attention_kv_heads(a.q, k_base, v_base, a.attn, a.scores, seq, n_past, nh, nkv, hd, scale,
-                               h, h + 1);
-      }
+      attend(m, a.q, NULL, l, k_base, v_base, a.attn, a.scores, seq, total, n_past, 0, scale);
     }
     mm(m, &w->wo, a.attn, a.h, seq, a.xq);
     add_rows(a.x, a.h, seq * d);
