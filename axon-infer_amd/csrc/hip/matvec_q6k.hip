@@ -30,13 +30,13 @@
 #include <atomic>
 #include "common.h"
 #include "matvec.h"
+#include "q6k_rows.h"
 #include <type_traits>
 
 namespace axon_hip {
 
 namespace {
 
-constexpr uint32_t kQ6MaxRows = 8;  // activation rows per workgroup of the planar kernel
 constexpr uint32_t kChainMaxOut = 2048;  // one activation row up to this many outputs: the chain kernel
 
 constexpr int kThreads = 256;  // rows per workgroup
@@ -995,51 +995,29 @@ int matvec_q6k_planar_launch(MatvecArgs& a, uint32_t n_in) {
     }
     if (ok) return check_launch("q6k_planar_chain");
   }
-  // Whole chunks of activation rows on the matrix cores where they give the chip its waves of 64
-  // output rows (two per SIMD for 32-row chunks, one for 16-row ones); the rows left over, and short
-  // matrices, on the vector ALU below. 128256 x 2048, us: 9 rows 170 there against 177 in one 16-row
-  // chunk, 12 rows 188 / 177, 16 + 4 rows 316 / 258, 24 rows 328 / 299 in one 32-row chunk (106305 x 1536 at 23: 223 / 231); 64000 rows
-  // (1000 waves) at 16 rows 128 / 110, 32000 rows at 16 rows 79 / 110 and at 32 rows 127 / 112.
-  {
-    const uint32_t waves = static_cast<uint32_t>(ceil_div(n_out, 64));
-    const uint32_t blocks = static_cast<uint32_t>(ceil_div(n_out, 256));
-    const float* x = reinterpret_cast<const float*>(a.xq);
+  // Chunks of activation rows on the matrix cores where they are the faster ones, the rows left over on
+  // the vector ALU below.
+  const Q6kRowsPlan plan = q6k_rows_plan(a.m, n_out, device_cus());
+  auto take = [&](auto kernel, uint32_t chunks, uint32_t rows) {
+    if (chunks == 0) return;
     MatvecArgs g = a;
-    auto take = [&](auto kernel, uint32_t chunks, uint32_t rows) {
-      g.m = std::min(a.m, chunks * rows);
-      launch(kernel, dim3(chunks, blocks), dim3(256), 0, g, n_in, col_bytes, g.m);
-      a.m -= g.m;
-      x += static_cast<size_t>(g.m) * n_in;
-      a.xq = reinterpret_cast<const uint8_t*>(x);
-      a.seg[0].y += static_cast<size_t>(g.m) * a.seg[0].y_stride;
-      g = a;
-    };
-    const uint32_t c32 = a.m / 32 + (a.m % 32 >= 24 ? 1 : 0);
-    if (blocks <= 65535 && static_cast<uint64_t>(c32) * waves >= 1536) take(q6k_planar_mfma_kernel<32>, c32, 32);
-    const uint32_t c16 = a.m / 16 + (a.m % 16 >= 10 ? 1 : 0);
-    // (With one wave per SIMD only where no rows are left over: 64000 rows at 24, 177 / 185 us.)
-    if (blocks <= 65535 && static_cast<uint64_t>(c16) * waves >= (c16 * 16 >= a.m ? 896 : 1536))
-      take(q6k_planar_mfma_kernel<16>, c16, 16);
-    if (a.m == 0) return check_launch("q6k_planar_mfma");
-  }
-  // Activation rows per workgroup: up to kQ6MaxRows (each lane then runs that many chains, and
-  // every weight slice is read once per that many rows), but fewer while that leaves under 1024
-  // waves of 64 rows: a lane's chains run one element after another, so a short matrix needs
-  // the rows spread over more waves more than it needs fewer weight reads. One launch covers
-  // every row, in chunks of equal size (20 rows: 7, 7 and 6 rather than 8, 8 and 4, whose last
-  // chunk would run eight chains per lane for four rows).
-  uint32_t mm = 1;
-  while (mm < kQ6MaxRows && mm < a.m) mm *= 2;
-  while (mm > 1 && ceil_div(a.m, mm) * ceil_div(n_out, 64) < 1024) mm /= 2;
-  mm = static_cast<uint32_t>(ceil_div(a.m, ceil_div(a.m, mm)));
+    g.m = std::min(a.m, chunks * rows);
+    launch(kernel, dim3(chunks, static_cast<uint32_t>(ceil_div(n_out, 256))), dim3(256), 0, g, n_in, col_bytes, g.m);
+    a.m -= g.m;
+    a.xq += static_cast<size_t>(g.m) * n_in * sizeof(float);
+    a.seg[0].y += static_cast<size_t>(g.m) * a.seg[0].y_stride;
+  };
+  take(q6k_planar_mfma_kernel<32>, plan.c32, 32);
+  take(q6k_planar_mfma_kernel<16>, plan.c16, 16);
+  if (a.m == 0) return check_launch("q6k_planar_mfma");
+  // The rest in one launch.
+  const Q6kLaneRows rows = q6k_lane_rows(a.m, n_out);
+  const uint32_t mm = rows.mm;
   const size_t lds = 0;
-  const uint32_t chunks = static_cast<uint32_t>(ceil_div(a.m, mm));
-  // 256 rows per workgroup when that still gives a workgroup per CU, else 64.
-  const bool wide = ceil_div(n_out, 256) * chunks >= 256;
-  const uint32_t th = wide ? 256 : 64;
-  const uint32_t blocks = static_cast<uint32_t>(ceil_div(n_out, th));
+  const bool wide = rows.wide;
+  const uint32_t blocks = static_cast<uint32_t>(ceil_div(n_out, wide ? 256 : 64));
   if (blocks > 65535) return fail(kUnsupported, "matmul_q6_k_planar: %u output rows", n_out);
-  const dim3 grid(chunks, blocks);
+  const dim3 grid(rows.chunks, blocks);
   const uint32_t m_total = a.m;
 #define AXON_Q6P(MM_)                                                                                       \
   case MM_:                                                                                                 \

@@ -286,12 +286,14 @@ def test_model_logits_unchanged_by_the_repack(H, tmp_path_factory):
 
 
 @pytest.mark.parametrize("n_rows,n_out,n_in", [
-    (10, 57409, 256),   # one 16-row chunk with 6 rows missing; the last wave holds one output row
+    (12, 98305, 256),   # one 16-row chunk with 4 rows missing; the last wave holds one output row
     (16, 98305, 512),   # a whole 16-row chunk
     (19, 98400, 256),   # 16 rows and 3 on the vector ALU
+    (30, 98305, 512),   # one 32-row chunk with 2 rows missing
     (32, 98305, 256),   # a whole 32-row chunk
-    (55, 98310, 512),   # two 32-row chunks, 9 rows missing
-    (70, 98310, 256),   # two 32-row chunks and 6 rows
+    (39, 98310, 256),   # 32 rows and 7
+    (55, 98310, 512),   # three 16-row chunks and 7 rows
+    (83, 57409, 256),   # two 32-row chunks, one of 16 and 3 rows
 ])
 def test_planar_many_rows(H, o, n_rows, n_out, n_in):
     """The matrix-core kernels' chunks and left-over rows, with strided outputs: the same rows in
