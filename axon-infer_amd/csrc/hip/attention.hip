@@ -14,6 +14,7 @@
 //
 // The workgroup's query heads share one kv head, so every K and V row is read from HBM once
 // per query row. Scores live in LDS when they fit, otherwise in a global scratch.
+#include <type_traits>
 #include "common.h"
 #include "elementwise.h"
 
@@ -760,6 +761,9 @@ __host__ __device__ inline size_t tile_lds(uint32_t max_vis) {
 }
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+// Four dwords in memory, aligned to a half and to a float.
+typedef uint32_t Words2 __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t Words4 __attribute__((ext_vector_type(4), aligned(4)));
 
 // Sixteen 4 x 4 outer products: rows the four values that block K of a holds (lanes 4 K .. 4 K + 3),
 // columns the four lanes of each block of b. Lane l's element v: a[4 K + v] * b[l].
@@ -790,8 +794,12 @@ __device__ __forceinline__ void for_each_index(F f) {
   }
 }
 
+// (Four waves per SIMD: two workgroups of 32 pairs share a CU as long as their LDS allows it, up to
+// about 400 positions. With 189 registers for the fp16 cache, which the direct loads once took, it was
+// one: 270 rows of 32 / 8 heads behind 218 positions 61 -> 55.5 us, 56 in the blocked kernel. The 16-pair
+// form is taken where its LDS leaves one workgroup per CU anyway.)
 template <bool F16, uint32_t G, uint32_t R>
-__global__ __launch_bounds__((64 * tile_waves<G, R>()), 2) void attention_tile_kernel(AttnArgs a, uint32_t n_rows) {
+__global__ __launch_bounds__((64 * tile_waves<G, R>()), (G * R == 32 ? 4 : 2)) void attention_tile_kernel(AttnArgs a, uint32_t n_rows) {
   constexpr uint32_t kPairs = G * R, W = tile_waves<G, R>();
   constexpr uint32_t es = F16 ? 2 : 4;
   constexpr uint32_t kStage = stage_bytes_of<F16>();
@@ -881,10 +889,25 @@ __global__ __launch_bounds__((64 * tile_waves<G, R>()), 2) void attention_tile_k
     for (uint32_t k = 0; k < 4; ++k) qa[k] = q[16 * k];
   }
 
+  // Four dwords of a K row in float.
+  auto widen = [](const auto& u, float* k) {
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+      if constexpr (F16) {
+        k[2 * i] = half_value(u[i] & 0xffffu);
+        k[2 * i + 1] = half_value(u[i] >> 16);
+      } else {
+        k[i] = __uint_as_float(u[i]);
+      }
+    }
+  };
   // Scores of 64 positions against the wave's pairs: half the dims at a time, in order.
   float m[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
   f32x4 dot = {0.0f, 0.0f, 0.0f, 0.0f};
-  auto add_half = [&]<int HALF>(const float (&kr)[32]) {
+  auto add_half = [&]<int HALF>(const auto (&w)[kChunks]) {
+    float kr[32];
+#pragma unroll
+    for (uint32_t c = 0; c < kChunks; ++c) widen(w[c], kr + 32 / kChunks * c);
     f32x4 p[32];
     for_each_index<0, 32>([&]<int D>() { p[D] = outer4<D % 16>(qa[2 * HALF + D / 16], kr[D]); });
 #pragma unroll
@@ -942,24 +965,12 @@ __global__ __launch_bounds__((64 * tile_waves<G, R>()), 2) void attention_tile_k
         __syncthreads();  // everyone's copies of this stage; the one before the last has been read
         if (st + 2 < n_stages) copy_k(ksrc, st + 2);
         if (kStagePos * (s >> 1) >= wmax) return;
-        const uint4* row = reinterpret_cast<const uint4*>(lds_tile + (st % kStages) * kStage) + lane * kChunks;
+        const u32x4* row = reinterpret_cast<const u32x4*>(lds_tile + (st % kStages) * kStage) + lane * kChunks;
         const uint32_t sw = swizzle(lane);
-        float kr[32];
+        u32x4 w[kChunks];
 #pragma unroll
-        for (uint32_t c = 0; c < kChunks; ++c) {
-          const uint4 u = row[c ^ sw];
-          const uint32_t w4[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-          for (uint32_t k = 0; k < 4; ++k) {
-            if constexpr (F16) {
-              kr[8 * c + 2 * k] = half_value(w4[k] & 0xffffu);
-              kr[8 * c + 2 * k + 1] = half_value(w4[k] >> 16);
-            } else {
-              kr[4 * c + k] = __uint_as_float(w4[k]);
-            }
-          }
-        }
-        add_half.template operator()<HALF>(kr);
+        for (uint32_t c = 0; c < kChunks; ++c) w[c] = row[c ^ sw];
+        add_half.template operator()<HALF>(w);
         if constexpr (HALF == 1) store_scores(kStagePos * (s >> 1), R);
       };
       half.template operator()<0>();
@@ -982,35 +993,26 @@ __global__ __launch_bounds__((64 * tile_waves<G, R>()), 2) void attention_tile_k
         n = k == i ? nv[k] : n;
       }
       if (!mine) continue;
-      const bool vec = aligned(off);
+      // Half the dims of position j0 + lane (past the last: of the last) from memory. A row starts on a
+      // whole element, which is all a vector load asks for. From an fp16 cache a half ahead of its use
+      // (283 rows of 32 / 4 heads at about 310 positions 90 -> 78 us); two float halves leave the
+      // scheduler no registers for the shared path (1.7 % slower there).
+      typedef std::conditional_t<F16, Words2, Words4> Words;
+      auto fetch = [&](uint32_t j0, uint32_t half, Words (&w)[kChunks]) {
+        const size_t e = static_cast<size_t>(off) + static_cast<size_t>(min(j0 + lane, n - 1)) * kv_row + static_cast<size_t>(g) * 64 + 32 * half;
+        const Words* row = reinterpret_cast<const Words*>(static_cast<const uint8_t*>(a.kv) + e * es);
+#pragma unroll
+        for (uint32_t c = 0; c < kChunks; ++c) w[c] = row[c];
+      };
+      Words lo[kChunks], hi[kChunks];
+      if (F16 && n > 0) fetch(0, 0, lo);
       for (uint32_t j0 = 0; j0 < n; j0 += 64) {
-        const size_t e = static_cast<size_t>(off) + static_cast<size_t>(min(j0 + lane, n - 1)) * kv_row + static_cast<size_t>(g) * 64;
-        auto half = [&]<int HALF>() {
-          float kr[32];
-          if (!vec) {
-#pragma unroll
-            for (uint32_t d = 0; d < 32; ++d) kr[d] = kv_at<F16>(a.kv, e + 32 * HALF + d);
-          } else {
-            const uint4* row = reinterpret_cast<const uint4*>(static_cast<const uint8_t*>(a.kv) + (e + 32 * HALF) * es);
-#pragma unroll
-            for (uint32_t c = 0; c < kChunks; ++c) {
-              const uint4 u = row[c];
-              const uint32_t w4[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-              for (uint32_t k = 0; k < 4; ++k) {
-                if constexpr (F16) {
-                  kr[8 * c + 2 * k] = half_value(w4[k] & 0xffffu);
-                  kr[8 * c + 2 * k + 1] = half_value(w4[k] >> 16);
-                } else {
-                  kr[4 * c + k] = __uint_as_float(w4[k]);
-                }
-              }
-            }
-          }
-          add_half.template operator()<HALF>(kr);
-        };
-        half.template operator()<0>();
-        half.template operator()<1>();
+        if constexpr (F16) fetch(j0, 1, hi);
+        else fetch(j0, 0, lo);
+        add_half.template operator()<0>(lo);
+        if constexpr (F16) fetch(j0 + 64, 0, lo);
+        else fetch(j0, 1, hi);
+        add_half.template operator()<1>(hi);
         store_scores(j0, i);
       }
     }
