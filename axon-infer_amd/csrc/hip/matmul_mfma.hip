@@ -17,6 +17,7 @@
 // 16-row activation tiles per wave), K staged through LDS 16 blocks at a time.
 #include "common.h"
 #include "matvec.h"
+#include "wide_tiles.h"
 
 #include <type_traits>
 #include <utility>
@@ -1303,7 +1304,6 @@ bool matmul_q8_rows_fits(int type, const MatvecArgs& a, bool many_rows) {
 }
 
 constexpr uint32_t kDecodeTileWg = 256;  // workgroups a decode matrix needs for the tile kernel
-constexpr uint32_t kWideMinBlocks = 48;  // blocks per row from which the largest tiles pay
 
 // From 128 tiles of 64 weight rows (33..64 rows, Q4_0): 8192 x 2048 24.4 -> 15.8 us, 9728 x 896
 // 20.7 -> 10.3, 16384 x 2048 46.0 -> 20.7; at 48 tiles and fewer the rows kernel stays ahead.
@@ -1361,13 +1361,12 @@ int matmul_q8_swiglu_launch(int type, MatvecArgs& a) {
   return wide_launch<16, 4, 4, 8, true>(type, a);
 }
 
-// The tile by how many workgroups it gives (two fit a CU): the largest that still fills the chip.
-// Measured at Q4_0, K = 2048, us: 64 x 128 / 64 x 64 tiles of 32 x 32 sums, 32 x 64 / 32 x 32 tiles of
-// 16 x 16 sums (the 16 x 16 kernel these replaced in brackets):
+// The tile of the least estimated time (wide_tiles.h). Measured at Q4_0, K = 2048, us: 64 x 128 / 64 x 64
+// tiles of 32 x 32 sums, 32 x 64 / 32 x 32 tiles of 16 x 16 sums (the 16 x 16 kernel these replaced in
+// brackets):
 //   512 x 16384  67 / 72 / 115 / 118 (99)     256 x 5632  29 / 23 / 26 / 27 (30)
 //   512 x 5632   35 / 31 / 44 / 45 (49)       512 x 2048  29 / 20 / 17 / 20 (19)
 //   512 x 3072   29 / 23 / 26 / 27 (29)       128 x 2048  28 / 19 / 13 / 10 (15)
-// Rows of fewer than kWideMinBlocks blocks keep to the smaller tile (896 x 9728 at 512 rows 31 / 25).
 int matmul_q8_tile_launch(int type, MatvecArgs& a) {
   if (!matmul_q8_rows_fits(type, a, true)) return fail(kUnsupported, "matmul tile: shape or alignment");
   auto workgroups = [&](uint32_t tm, uint32_t tn) {
@@ -1377,10 +1376,14 @@ int matmul_q8_tile_launch(int type, MatvecArgs& a) {
   };
   // 128 weight rows behind one buffer descriptor, whose size is 31 bits.
   const bool sized = static_cast<uint64_t>(a.nb) * kBytesQ8_0 * 128 < (uint64_t(1) << 31);
-  if (workgroups(64, 128) >= 512 && a.nb >= kWideMinBlocks && sized) return wide_launch<32, 2, 2, 8>(type, a);
-  if (workgroups(64, 64) >= 320) return wide_launch<32, 2, 1, 8>(type, a);
-  if (workgroups(32, 64) >= 512) return wide_launch<16, 2, 2, 16>(type, a);
-  return wide_launch<16, 2, 1, 16>(type, a);
+  const uint64_t counts[kWideTiles] = {workgroups(64, 128), workgroups(64, 64), workgroups(32, 64), workgroups(32, 32)};
+  const WideType kind = type == Q8_0 ? kWideQ8_0 : type == Q4_0 ? kWideQ4_0 : kWideQ4_1;
+  switch (wide_tile(kind, a.nb, counts, device_cus(), sized)) {
+  case kTile64x128: return wide_launch<32, 2, 2, 8>(type, a);
+  case kTile64x64: return wide_launch<32, 2, 1, 8>(type, a);
+  case kTile32x64: return wide_launch<16, 2, 2, 16>(type, a);
+  default: return wide_launch<16, 2, 1, 16>(type, a);
+  }
 }
 
 int matmul_q8_rows_launch(int type, MatvecArgs& a) {

@@ -95,6 +95,8 @@ uint32_t q6k_planar_argmax_parts(uint32_t n_out);
 // Test hook: 0 chooses the one-row kernel by shape; 1 the one-lane-per-row kernel, 2 the
 // products-then-chains kernel (where its LDS fits), 3 the streamed-ring kernel.
 void matvec_q6k_force_path(int path);
+// Compute units of the current device.
+uint32_t device_cus();
 // q|k|v of 1..kRowsMaxM rows on the few-rows MFMA kernel with the RowsRope epilogue
 // (kUnsupported, nothing launched, where matmul_q8_rows_fits refuses the shape).
 int matmul_q8_rows_rope_launch(int type, MatvecArgs& a, const RowsRope& rp);
