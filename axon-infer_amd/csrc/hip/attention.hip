@@ -1156,21 +1156,39 @@ bool try_tile(const AttnArgs& a, uint32_t n_rows) {
   return true;
 }
 
-// Workgroups of 32 pairs where they leave one per CU and their scores fit; else of 16 where the
-// blocked kernel's do not (with both, the blocked kernel is the faster one: 128 rows behind 700
-// positions 58 against 66 us) and two workgroups per CU are there: its single rows spread wider below
-// that (32 / 4 heads: 163 rows behind 885 positions, 328 workgroups, 88 against 135 us, 195 behind
-// 1001, 392 workgroups, 139 against 155). Groups of 3 and 7 heads, whose waves would span rows, stay with the
-// blocked kernel (512 rows of 14 / 2 heads: 53 us either way).
+// Workgroups of 16 pairs while two of them share a CU (up to 832 positions with a float cache, 1024
+// with an fp16 one) and there are two per CU: the last round of fewer, larger workgroups stands emptier,
+// and rows of a batch that lie further apart wait less for each other. 16 against 32 pairs, us: 264 rows
+// of 32 / 8 heads behind 60 positions, fp16, 31.8 / 39.0, 280 behind 298 73 / 77; a batch of 292 rows of
+// up to 349 positions, float, 67 / 70 (blocked kernel: 74), of 297 rows of up to 461 85 / 108 (87). Two
+// workgroups of 32 pairs on most CUs are the faster ones with a float cache, whose K and V they read
+// half as often (253 rows of 64 / 8 heads 32.5 / 35.0).
+// Else 32 pairs where they leave one workgroup per CU and their scores fit; else 16 where the blocked
+// kernel's do not (with both, the blocked kernel is the faster one: 128 rows behind 700 positions 58
+// against 66 us) and two workgroups per CU are there: its single rows spread wider below that (32 / 4
+// heads: 163 rows behind 885 positions, 328 workgroups, 88 against 135 us, 195 behind 1001, 392
+// workgroups, 139 against 155).
+// Float batches of more than 250 sequences past 832 positions run at 0.73 to 2 times the blocked
+// kernel's speed, mostly faster: whether the rows share a span is not known here.
+// Groups of 3 and 7 heads, whose waves would span rows, stay with the blocked kernel (512 rows of 14 / 2
+// heads: 53 us either way).
 template <uint32_t G>
 bool launch_tile_g(const AttnArgs& a, uint32_t n_rows) {
+  constexpr size_t kCuLds = 160 * 1024, kOwnLds = 256;  // a CU's, and the kernel's own table
+  auto workgroups = [&](uint32_t rows) { return static_cast<size_t>((n_rows + rows - 1) / rows) * a.n_kv; };
+  auto two_fit = [&]<uint32_t R>() {
+    return 2 * ((a.f16 ? tile_lds<true, G, R>(a.max_vis) : tile_lds<false, G, R>(a.max_vis)) + kOwnLds) <= kCuLds;
+  };
   auto attempt = [&]<uint32_t R>() {
     constexpr size_t kLeast = G * R == 32 ? kTileMinWorkgroups : 2 * kTileMinWorkgroups;
-    if (static_cast<size_t>((n_rows + R - 1) / R) * a.n_kv < kLeast) return false;
+    if (workgroups(R) < kLeast) return false;
     return a.f16 ? try_tile<true, G, R>(a, n_rows) : try_tile<false, G, R>(a, n_rows);
   };
-  if (attempt.template operator()<32 / G>()) return true;
-  return block_lds(16, a.max_vis) > kBlockMaxLds && attempt.template operator()<16 / G>();
+  constexpr uint32_t kMany = 32 / G, kFew = 16 / G;  // rows of a workgroup
+  const bool many_pair = !a.f16 && two_fit.template operator()<kMany>() && 2 * workgroups(kMany) >= 3 * kTileMinWorkgroups;
+  if (!many_pair && two_fit.template operator()<kFew>() && attempt.template operator()<kFew>()) return true;
+  if (attempt.template operator()<kMany>()) return true;
+  return block_lds(16, a.max_vis) > kBlockMaxLds && attempt.template operator()<kFew>();
 }
 
 // The tiled kernel for whole-head launches of 64-dim heads and kv groups of 4 or 8 query heads;

@@ -1,7 +1,8 @@
 """Many-row attention with its products on the matrix cores (kv groups of 4 and 8 heads), where it
 can go wrong: rows that end inside a block, positions around the 64- and 32-position stages, the
 16-pair form of long contexts, spans that are not 16-byte aligned, blocks whose rows belong to
-different sequences, and values that are not finite past a row's own positions. Bit for bit against
+different sequences, and values that are not finite past a row's own positions. Workgroups take 16 (row, head)
+pairs where there are 512 of them and two share a CU, else 32 where there are 256. Bit for bit against
 the oracle, the Q8_0 blocks of the outputs too."""
 import ctypes as C
 
@@ -81,28 +82,40 @@ def check(o, h, chunk, past, decode, n_head, n_kv, f16, shift=0, poison=False, s
 
 @pytest.mark.parametrize("f16", [False, True])
 @pytest.mark.parametrize("chunk,past,n_head,n_kv", [
-    (250, 0, 32, 8),     # a last block of two rows; contexts from one position up
-    (257, 63, 32, 8),    # a last block of one row, contexts across the first K stage
-    (505, 31, 32, 4),    # groups of 8 heads: four rows per workgroup
+    (250, 0, 32, 8),     # 32 pairs; a last block of two rows; contexts from one position up
+    (385, 63, 32, 8),    # a last block of one row, contexts across the first K stage
+    (257, 63, 32, 8),    # 16 pairs: a last block of one row
+    (505, 31, 32, 4),    # groups of 8 heads: two or four rows per workgroup
     (128, 1100, 32, 8),  # 16 pairs' LDS, too few workgroups for them
     (128, 1030, 64, 8),  # the same with groups of 8
     (64, 1100, 128, 32),  # both again at the 512 workgroups that 16 pairs ask for
     (64, 1030, 128, 16),
+    (256, 1500, 32, 4),  # rows too long for the blocked kernel's LDS: one per CU of 16 pairs, with a scratch
 ])
 def test_chunk(o, h, chunk, past, n_head, n_kv, f16):
     check(o, h, chunk, past, [], n_head, n_kv, f16)
 
 
-@pytest.mark.parametrize("f16", [False, True])
-def test_unaligned_span(o, h, f16):
-    check(o, h, 250, 20, [], 32, 8, f16, shift=1)
+# Either side of the last position at which two workgroups of 16 pairs share a CU, and of the last
+# that 32 pairs' scores fit.
+@pytest.mark.parametrize("f16,total", [(False, 832), (False, 833), (False, 1024), (False, 1025), (True, 1024), (True, 1025),
+                                       (True, 1152), (True, 1153)])
+def test_positions_at_the_edges_of_lds(o, h, f16, total):
+    check(o, h, 256, total - 256, [], 32, 8, f16)
 
 
 @pytest.mark.parametrize("f16", [False, True])
-@pytest.mark.parametrize("n_head,n_kv", [(32, 8), (64, 8)])
-def test_rows_of_other_sequences(o, h, n_head, n_kv, f16):
-    check(o, h, 243, 9, [1, 64, 65, 300, 17, 128, 33], n_head, n_kv, f16)
+@pytest.mark.parametrize("chunk", [250, 257])  # 32 pairs, 16 pairs
+def test_unaligned_span(o, h, chunk, f16):
+    check(o, h, chunk, 20, [], 32, 8, f16, shift=1)
+
+
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("chunk,n_head,n_kv", [(243, 32, 8), (254, 32, 8), (243, 64, 8), (120, 64, 8)])
+def test_rows_of_other_sequences(o, h, chunk, n_head, n_kv, f16):
+    check(o, h, chunk, 9, [1, 64, 65, 300, 17, 128, 33], n_head, n_kv, f16)
 
 
 def test_nothing_from_past_a_rows_positions(o, h):
-    check(o, h, 256, 15, [], 32, 8, False, poison=True)
+    check(o, h, 248, 15, [], 32, 8, False, poison=True)  # 32 pairs
+    check(o, h, 256, 15, [], 32, 8, False, poison=True)  # 16
