@@ -30,13 +30,11 @@
 // 151936 logits, k 40: 64 rows 100 -> 32 us, one row 76 -> 24, 64 rows of one value each 90 -> 56;
 // 32000 logits, 8 rows 45.6 -> 10.6; 128256 logits, k 256, 64 rows 140 -> 32. Most of the time
 // before was the sort below.
-// Rows where more than 1024 values lie above the bound, since the large ones fall to few threads,
-// go on to rounds: each thread keeps the four largest keys below a bound among its strided elements;
-// the 4096 kept keys are sorted in LDS (bitonic). Let M be the largest fourth key over the threads
-// that kept four. Every key above M is then among the kept ones (a thread's dropped keys lie below
-// its fourth), so the sorted keys above M are the row's next keys in order and are taken. The thread
-// that holds M kept three keys above it, so a round takes at least three. Such a row pays for the
-// sweeps before (64 rows of 151936 with 30 of each 1024 columns raised: 241 -> 282 us).
+// Rows where more than 1024 values lie above the bound, since the large ones fall to few threads, find
+// their k-th largest value itself the same way, a sweep for each of the four digits over the values
+// above the bound (at most a quarter of the row: 768 threads hold none), and go on as rows of many
+// equal values do. 64 rows with 30 of each 1024 columns raised, us: 151936 logits, k 40, 259 by rounds of
+// sorting each thread's four largest keys, 162 here; 128256 logits, k 256, 751 and 154.
 #include "common.h"
 #include "elementwise.h"
 
@@ -106,48 +104,51 @@ __global__ __launch_bounds__(256) void repeat_penalty_kernel(float* __restrict__
 }
 
 constexpr uint32_t kTopKThreads = 1024;
-constexpr uint32_t kTopKKeep = 4;
-constexpr uint32_t kTopKKeys = kTopKThreads * kTopKKeep;
 constexpr uint32_t kTopKUnroll = 8;     // loads in flight per thread in a sweep
-constexpr uint32_t kTopKList = 1024;    // candidates that the threshold path takes
+constexpr uint32_t kTopKList = 1024;    // candidates that one gather takes
+constexpr uint32_t kTopKKeys = kMaxTopK + kTopKThreads;  // k keys and one more step's of equal values
 
 __global__ __launch_bounds__(kTopKThreads) void topk_rows_kernel(const float* __restrict__ x, uint32_t n, size_t stride,
                                                                  uint32_t k, float* __restrict__ out_logit,
                                                                  int32_t* __restrict__ out_id) {
+  static_assert(kTopKList <= kTopKKeys, "a gather's keys fit");
   __shared__ uint64_t keys[kTopKKeys];
-  __shared__ uint64_t red[kTopKThreads / 64];
   __shared__ uint32_t taken;
-  const uint32_t r = blockIdx.x;
-  const uint32_t t = threadIdx.x;
+  __shared__ uint32_t pick[2];  // a digit, and how many values are still wanted within it
+  uint32_t* hist = reinterpret_cast<uint32_t*>(keys);
+  const uint32_t r = blockIdx.x, t = threadIdx.x;
   const float* row = x + static_cast<size_t>(r) * stride;
   float* ol = out_logit + static_cast<size_t>(r) * k;
   int32_t* oi = out_id + static_cast<size_t>(r) * k;
 
-  // By a threshold, where that leaves few enough candidates (see above).
-  {
-    float m = -INFINITY;  // fmaxf passes NaN over
+  // This thread's elements of the row, kTopKUnroll at a time, past the end as `pad`; stops early on false.
+  auto sweep = [&](float pad, auto take) {
     for (uint32_t j0 = t; j0 < n; j0 += kTopKUnroll * kTopKThreads) {
       float v[kTopKUnroll];
 #pragma unroll
       for (uint32_t i = 0; i < kTopKUnroll; ++i) {
         const uint32_t j = j0 + i * kTopKThreads;
-        v[i] = j < n ? row[j] : -INFINITY;
+        v[i] = j < n ? row[j] : pad;
       }
-#pragma unroll
-      for (uint32_t i = 0; i < kTopKUnroll; ++i) m = fmaxf(m, v[i]);
+      if (!take(j0, v)) break;
     }
-    const uint32_t mo = static_cast<uint32_t>(argmax_key(m, 0) >> 32);
-    uint32_t* hist = reinterpret_cast<uint32_t*>(keys);
-    __shared__ uint32_t pick[2];  // a digit, and how many maxima are still wanted within it
+  };
+  // The order of a value among values, and the value (negative zero as zero).
+  auto order = [](float v) { return static_cast<uint32_t>(argmax_key(v, 0) >> 32); };
+  // The k-th largest of the values that fill(d, prefix) counts into hist by digit d (8 bits, the upper
+  // one first), those whose larger digits are prefix.
+  auto kth = [&](auto fill) {
     uint32_t prefix = 0, want = k;
-#pragma unroll
-    for (int d = 0; d < 4; ++d) {  // digits of 8 bits, the upper one first
+#pragma unroll 1
+    for (int d = 0; d < 4; ++d) {
       if (t < 256) hist[t] = 0;
       __syncthreads();
-      if (d == 0 || (mo >> ((32 - 8 * d) & 31)) == prefix) atomicAdd(&hist[(mo >> (24 - 8 * d)) & 0xffu], 1u);
+      fill([&](uint32_t o) {
+        if (d == 0 || (o >> ((32 - 8 * d) & 31)) == prefix) atomicAdd(&hist[(o >> (24 - 8 * d)) & 0xffu], 1u);
+      });
       __syncthreads();
       if (t < 64) {
-        // Lane t holds digits 4 t .. 4 t + 3; above: the maxima of larger digits.
+        // Lane t holds digits 4 t .. 4 t + 3; above: the values of larger digits.
         uint32_t c[4], own = 0;
 #pragma unroll
         for (uint32_t i = 0; i < 4; ++i) own += c[i] = hist[4 * t + i];
@@ -172,146 +173,76 @@ __global__ __launch_bounds__(kTopKThreads) void topk_rows_kernel(const float* __
       want = pick[1];
       __syncthreads();
     }
-    const float bound_v = __uint_as_float((prefix & 0x80000000u) ? prefix & 0x7fffffffu : ~prefix);
-    // Gathers the keys of values that reach the bound (or lie above it); stops, with more than
-    // kTopKList counted, once they are too many.
-    auto gather = [&](bool ties) -> uint32_t {
-      if (t == 0) taken = 0;
-      __syncthreads();
-      for (uint32_t j0 = t; j0 < n; j0 += kTopKUnroll * kTopKThreads) {
-        float v[kTopKUnroll];
-#pragma unroll
-        for (uint32_t i = 0; i < kTopKUnroll; ++i) {
-          const uint32_t j = j0 + i * kTopKThreads;
-          v[i] = j < n ? row[j] : __uint_as_float(0x7fc00000u);
-        }
-#pragma unroll
-        for (uint32_t i = 0; i < kTopKUnroll; ++i) {
-          if (ties ? v[i] >= bound_v : v[i] > bound_v) {
-            const uint32_t at = atomicAdd(&taken, 1u);
-            if (at < kTopKList) keys[at] = argmax_key(v[i], j0 + i * kTopKThreads);
-          }
-        }
-        if (*static_cast<volatile uint32_t*>(&taken) > kTopKList) break;
-      }
-      __syncthreads();
-      const uint32_t got = taken;
-      __syncthreads();
-      return got;
-    };
-    uint32_t count = gather(true);
-    bool fits = count <= kTopKList;
-    if (!fits) {
-      // Many equal values at the bound: those above it, then, where they are fewer than k, the first
-      // of the equal ones, 1024 elements at a time in index order until k keys are there.
-      count = gather(false);
-      fits = count <= kTopKList;
-      static_assert(kMaxTopK + kTopKThreads <= kTopKKeys, "k keys and one more step's fit");
-      if (t == 0) taken = count;
-      __syncthreads();
-      for (uint32_t j0 = 0; count < k && j0 < n; j0 += kTopKThreads) {
-        const uint32_t j = j0 + t;
-        if (j < n && row[j] == bound_v) keys[atomicAdd(&taken, 1u)] = argmax_key(bound_v, j);
-        __syncthreads();
-        count = taken;
-        __syncthreads();
-      }
-    }
-    if (fits) {
-      for (uint32_t i = t; i < count; i += kTopKThreads) {
-        const uint64_t key = keys[i];
-        uint32_t rank = 0;
-        for (uint32_t q = 0; q < count; ++q) rank += keys[q] > key ? 1u : 0u;
-        if (rank < k) {
-          const uint32_t id = ~static_cast<uint32_t>(key & 0xffffffffu);
-          ol[rank] = row[id];
-          oi[rank] = static_cast<int32_t>(id);
-        }
-      }
-      for (uint32_t i = count + t; i < k; i += kTopKThreads) {  // fewer than k non-NaN values
-        ol[i] = 0.0f;
-        oi[i] = -1;
-      }
-      return;
-    }
-  }
+    return __uint_as_float((prefix & 0x80000000u) ? prefix & 0x7fffffffu : ~prefix);
+  };
 
-  uint32_t got = 0;
-  uint64_t bound = ~0ull;  // above every key
-  for (;;) {
-    uint64_t c0 = 0, c1 = 0, c2 = 0, c3 = 0;  // descending; 0 is below every key
-    for (uint32_t j = t; j < n; j += kTopKThreads) {
-      const float v = row[j];
-      if (v != v) continue;
-      const uint64_t key = argmax_key(v, j);
-      if (key >= bound || key <= c3) continue;
-      if (key > c2) {
-        c3 = c2;
-        if (key > c1) {
-          c2 = c1;
-          if (key > c0) {
-            c1 = c0;
-            c0 = key;
-          } else {
-            c1 = key;
-          }
-        } else {
-          c2 = key;
-        }
-      } else {
-        c3 = key;
-      }
-    }
-    const uint64_t m = max_key_wave(c3);
-    if ((t & 63) == 0) red[t >> 6] = m;
-    keys[kTopKKeep * t] = c0;
-    keys[kTopKKeep * t + 1] = c1;
-    keys[kTopKKeep * t + 2] = c2;
-    keys[kTopKKeep * t + 3] = c3;
+  float m = -INFINITY;  // fmaxf passes NaN over
+  sweep(-INFINITY, [&](uint32_t, const float (&v)[kTopKUnroll]) {
+#pragma unroll
+    for (uint32_t i = 0; i < kTopKUnroll; ++i) m = fmaxf(m, v[i]);
+    return true;
+  });
+  float bound = kth([&](auto count) { count(order(m)); });
+  // Gathers the keys of values that reach the bound (or lie above it); stops, with more than
+  // kTopKList counted, once they are too many.
+  auto gather = [&](bool ties) -> uint32_t {
     if (t == 0) taken = 0;
     __syncthreads();
-    // Bitonic sort, descending: 2048 compare-exchanges per stage, two per thread.
-    for (uint32_t size = 2; size <= kTopKKeys; size <<= 1) {
-      for (uint32_t half = size >> 1; half > 0; half >>= 1) {
+    sweep(__uint_as_float(0x7fc00000u), [&](uint32_t j0, const float (&v)[kTopKUnroll]) {
 #pragma unroll
-        for (uint32_t p = 0; p < 2; ++p) {
-          const uint32_t q = t + p * kTopKThreads;  // pair index
-          const uint32_t i = 2 * q - (q & (half - 1));
-          const uint32_t j = i + half;
-          const uint64_t a = keys[i], b = keys[j];
-          const bool desc = (i & size) == 0;
-          if (desc ? a < b : a > b) {
-            keys[i] = b;
-            keys[j] = a;
-          }
+      for (uint32_t i = 0; i < kTopKUnroll; ++i) {
+        if (ties ? v[i] >= bound : v[i] > bound) {
+          const uint32_t at = atomicAdd(&taken, 1u);
+          if (at < kTopKList) keys[at] = argmax_key(v[i], j0 + i * kTopKThreads);
         }
-        __syncthreads();
       }
-    }
-    uint64_t big_m = red[0];
-    for (uint32_t w = 1; w < kTopKThreads / 64; ++w) big_m = red[w] > big_m ? red[w] : big_m;
-    // g = the number of sorted keys above M (keys at or below M, zeros included, follow them).
+      return *static_cast<volatile uint32_t*>(&taken) <= kTopKList;
+    });
+    __syncthreads();
+    const uint32_t got = taken;
+    __syncthreads();
+    return got;
+  };
+  uint32_t count = gather(true);
+  if (count > kTopKList) {
+    // Many equal values at the bound, or many above it: in the latter case the bound moves up to the
+    // k-th largest value. Then those above it, and, where they are fewer than k, the first of the
+    // equal ones, 1024 elements at a time in index order until k keys are there.
+    count = gather(false);
+    if (count > kTopKList) {
+      const float low = bound;
+      bound = kth([&](auto add) {
+        if (m > low)
+          sweep(low, [&](uint32_t, const float (&v)[kTopKUnroll]) {
 #pragma unroll
-    for (uint32_t p = 0; p < kTopKKeep; ++p) {
-      const uint32_t i = kTopKKeep * t + p;
-      if (keys[i] > big_m && (i + 1 == kTopKKeys || keys[i + 1] <= big_m)) taken = i + 1;
+            for (uint32_t i = 0; i < kTopKUnroll; ++i)
+              if (v[i] > low) add(order(v[i]));
+            return true;
+          });
+      });
+      count = gather(false);
     }
+    if (t == 0) taken = count;
     __syncthreads();
-    const uint32_t g = taken;
-    const uint32_t take = min(g, k - got);
-    for (uint32_t i = t; i < take; i += kTopKThreads) {
-      const uint64_t key = keys[i];
-      const uint32_t id = ~static_cast<uint32_t>(key & 0xffffffffu);
-      ol[got + i] = row[id];
-      oi[got + i] = static_cast<int32_t>(id);
+    for (uint32_t j0 = 0; count < k && j0 < n; j0 += kTopKThreads) {
+      const uint32_t j = j0 + t;
+      if (j < n && row[j] == bound) keys[atomicAdd(&taken, 1u)] = argmax_key(bound, j);
+      __syncthreads();
+      count = taken;
+      __syncthreads();
     }
-    got += take;
-    // Done at k keys, or when no thread kept four (every remaining key was taken).
-    if (got == k || big_m == 0) break;
-    bound = keys[take - 1];
-    __syncthreads();
   }
-  for (uint32_t i = got + t; i < k; i += kTopKThreads) {  // fewer than k non-NaN values
+  for (uint32_t i = t; i < count; i += kTopKThreads) {
+    const uint64_t key = keys[i];
+    uint32_t rank = 0;
+    for (uint32_t q = 0; q < count; ++q) rank += keys[q] > key ? 1u : 0u;
+    if (rank < k) {
+      const uint32_t id = ~static_cast<uint32_t>(key & 0xffffffffu);
+      ol[rank] = row[id];
+      oi[rank] = static_cast<int32_t>(id);
+    }
+  }
+  for (uint32_t i = count + t; i < k; i += kTopKThreads) {  // fewer than k non-NaN values
     ol[i] = 0.0f;
     oi[i] = -1;
   }

@@ -332,6 +332,29 @@ def test_topk_rows_threshold_edges(H, n, k):
         assert np.array_equal(got_v[r].view(np.uint32), want_v.view(np.uint32)), r
 
 
+@pytest.mark.parametrize("n", [20000, 151936])
+@pytest.mark.parametrize("k", [1, 40, 91, 256])
+def test_topk_rows_large_values_with_few_threads(H, n, k):
+    """More than 1024 values above the bound, all in 90 of each 1024 columns: spread, equal, equal in
+    all but their last bits, zeros of both signs, infinities and NaN among them, negative ones."""
+    rng = np.random.default_rng(n + k)
+    few = np.arange(n) % 1024 < 90
+    bits = lambda base, width: (np.uint32(base) | rng.integers(0, width, n).astype(np.uint32)).view(np.float32)
+    spread = rng.standard_normal(n).astype(np.float32)
+    large = [spread + 50, np.full(n, 7, np.float32), bits(0x42480000, 3), bits(0x42480000, 1 << 16),
+             np.where(rng.random(n) < 0.5, np.float32(0.0), np.float32(-0.0)), spread + 50, -1 - np.abs(spread)]
+    large[5][rng.integers(0, n, 300)] = np.inf
+    large[5][rng.integers(0, n, 300)] = np.nan
+    x = np.stack([np.where(few, v, -100 - np.abs(spread)).astype(np.float32) for v in large])
+    dx, ol, oi = H.DeviceBuffer.of(x), H.DeviceBuffer(4 * len(x) * k), H.DeviceBuffer(4 * len(x) * k)
+    H.call("topk_rows", dx, n, len(x), n, k, ol, oi)
+    got_v, got_i = ol.download(np.float32).reshape(len(x), k), oi.download(np.int32).reshape(len(x), k)
+    for r in range(len(x)):
+        want_v, want_i = topk_reference(x[r], k)
+        assert np.array_equal(got_i[r], want_i), r
+        assert np.array_equal(got_v[r].view(np.uint32), want_v.view(np.uint32)), r
+
+
 def test_topk_rows_bounds(H):
     dx = H.DeviceBuffer.of(np.zeros(300, np.float32))
     out = H.DeviceBuffer(4 * 300)
