@@ -12,6 +12,12 @@ from helpers import BLOCK, Q8_0, call, oracle, ref
 QUANT_TYPES = ("q8_0", "q4_0", "q4_1")
 
 
+def same_bits(a, b) -> bool:
+    """Bit for bit, signs of zero too; a NaN equals any NaN."""
+    a, b = (np.ascontiguousarray(v, np.float32) for v in (a, b))
+    return a.shape == b.shape and bool(np.all((a.view(np.uint32) == b.view(np.uint32)) | (np.isnan(a) & np.isnan(b))))
+
+
 class CTable:
     """The oracle (prefix "ora_") or the reference build (prefix "ref_")."""
 

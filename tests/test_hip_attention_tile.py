@@ -41,14 +41,17 @@ def run(h, q, pool, k_off, v_off, n_vis, n_head, n_kv, f16):
     return out.download(np.float32).reshape(n, n_head, HD), outq.download(np.uint8)
 
 
-def check(o, h, chunk, past, decode, n_head, n_kv, f16, shift=0, poison=False, seed=1):
-    """A chunk of `chunk` rows behind `past` positions, then one row of each sequence in `decode`."""
+def check(o, h, chunk, past, decode, n_head, n_kv, f16, shift=0, poison=False, seed=1, change=None):
+    """A chunk of `chunk` rows behind `past` positions, then one row of each sequence in `decode`.
+    `change` alters the queries and the chunk's keys and values in place."""
     rng = np.random.default_rng(seed)
     seqs = [past + chunk] + list(decode)
     n = chunk + len(decode)
     row = n_kv * HD
     q = rng.standard_normal((n, n_head, HD)).astype(np.float32)
     kv = [(rng.standard_normal((m, row)).astype(np.float32), rng.standard_normal((m, row)).astype(np.float32)) for m in seqs]
+    if change is not None:
+        change(rng, q, *kv[0])
     if f16:
         kv = [(k.astype(np.float16), v.astype(np.float16)) for k, v in kv]
     want = np.zeros((n, n_head, HD), np.float32)
@@ -119,3 +122,19 @@ def test_rows_of_other_sequences(o, h, chunk, n_head, n_kv, f16):
 def test_nothing_from_past_a_rows_positions(o, h):
     check(o, h, 248, 15, [], 32, 8, False, poison=True)  # 32 pairs
     check(o, h, 256, 15, [], 32, 8, False, poison=True)  # 16
+
+
+def subnormal(rng, q, k, v):
+    """Rows whose products with the keys lie below the smallest normal float, rows whose scores lie so
+    far apart that most probabilities do, and values of every size."""
+    q[::4] *= np.float32(1e-37)
+    q[1::4] *= np.float32(1e-40)
+    q[2::4] *= np.float32(40)
+    k[:, ::2] *= np.float32(1e-3)
+    v *= (np.float32(10) ** rng.integers(-40, 1, v.shape)).astype(np.float32)
+
+
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("chunk", [248, 256])  # 32 pairs, 16 pairs
+def test_subnormal_products(o, h, chunk, f16):
+    check(o, h, chunk, 15, [], 32, 8, f16, change=subnormal)

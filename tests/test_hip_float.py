@@ -5,7 +5,7 @@ oracle."""
 import numpy as np
 import pytest
 
-from tables import CTable, HipTable, random_floats
+from tables import CTable, HipTable, random_floats, same_bits
 
 pytestmark = pytest.mark.gpu
 
@@ -49,7 +49,7 @@ def test_float_matmul_infinities_stay_in_their_row(o, h, kind):
     x[7 * n_in + 299] = np.inf
     x[17 * n_in] = np.nan
     want = o.matmul(kind, w, x, n_out, n_in, n_rows=n_rows)
-    assert np.array_equal(h.matmul(kind, w, x, n_out, n_in, n_rows=n_rows), want, equal_nan=True)
+    assert same_bits(h.matmul(kind, w, x, n_out, n_in, n_rows=n_rows), want)
 
 
 # Both row counts of a tile on whole and partial ones: 32 rows up to 16 rows of input, and from 256

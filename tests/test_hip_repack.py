@@ -17,7 +17,7 @@ import numpy as np
 import pytest
 
 from helpers import Q6_K
-from tables import CTable, HipTable, dequantize, random_floats, random_weights
+from tables import CTable, HipTable, dequantize, random_floats, random_weights, same_bits
 
 pytestmark = pytest.mark.gpu
 
@@ -315,6 +315,27 @@ def test_planar_many_rows(H, o, n_rows, n_out, n_in):
         m = min(8, n_rows - r0)
         part = H.DeviceBuffer(m * n_out * 4)
         H.call("matmul_q6_k_planar", planar, dx.at(r0 * n_in * 4), part, m, n_out, n_in, n_out)
-        assert np.array_equal(got[r0:r0 + m, :n_out], part.download(np.float32).reshape(m, n_out), equal_nan=True)
+        assert same_bits(got[r0:r0 + m, :n_out], part.download(np.float32).reshape(m, n_out))
     for r in (0, n_rows - 1):
-        assert np.array_equal(got[r, :n_out], o.matmul("q6_k", w, x[r], n_out, n_in), equal_nan=True)
+        assert same_bits(got[r, :n_out], o.matmul("q6_k", w, x[r], n_out, n_in))
+
+
+@pytest.mark.parametrize("n_rows", [12, 32])
+def test_planar_subnormal_products(H, o, n_rows):
+    """Activations and products below the smallest normal float through the matrix cores (one chunk of
+    16 and one of 32 rows), which are to keep them as the vector ALU does."""
+    n_out, n_in = 98305, 256
+    w = q6k_weights(n_out, n_in, 31)
+    planar, _ = repack(H, w, n_out, n_in)
+    rng = np.random.default_rng(32)
+    x = random_floats(n_rows * n_in, 33, 1.0).reshape(n_rows, n_in) * np.float32(1e-39)
+    x[rng.random(x.shape) < 0.5] *= np.float32(1e-4)
+    x[rng.random(x.shape) < 0.2] *= np.float32(0.1)
+    assert np.mean(np.abs(x) < np.finfo(np.float32).tiny) > 0.3
+    y = H.DeviceBuffer(n_rows * n_out * 4)
+    H.call("matmul_q6_k_planar", planar, H.DeviceBuffer.of(x), y, n_rows, n_out, n_in, n_out)
+    got = y.download(np.float32).reshape(n_rows, n_out)
+    for r in (0, 5, n_rows - 1):
+        want = o.matmul("q6_k", w, x[r], n_out, n_in)
+        assert 0.3 < np.mean((want != 0) & (np.abs(want) < np.finfo(np.float32).tiny))
+        assert same_bits(got[r], want), r

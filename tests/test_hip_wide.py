@@ -8,7 +8,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
-from tables import CTable, HipTable, QUANT_TYPES, random_floats, random_weights
+from tables import CTable, HipTable, QUANT_TYPES, random_floats, random_weights, same_bits
 
 pytestmark = pytest.mark.gpu
 
@@ -23,10 +23,6 @@ def h():
     return HipTable()
 
 
-def same(a, b):
-    return np.array_equal(np.asarray(a).view(np.uint32), np.asarray(b).view(np.uint32))
-
-
 def inputs(o, kind, m, n_out, n_in, seed=1):
     xq = np.concatenate([o.quantize_row_q8_0(random_floats(n_in, seed * 1000 + r, 3.0)) for r in range(m)])
     return random_weights(kind, n_out, n_in, seed), xq
@@ -38,9 +34,9 @@ def check(o, h, kind, w, xq, m, n_out, n_in):
     for r0 in range(0, m, 16):
         rows = min(16, m - r0)
         want = h.matmul(kind + "_q8", w, xq[r0 * nb:(r0 + rows) * nb], n_out, n_in, n_rows=rows)
-        assert np.array_equal(y[r0:r0 + rows].ravel(), want, equal_nan=True), f"rows from {r0}"
+        assert same_bits(y[r0:r0 + rows].ravel(), want), f"rows from {r0}"
     for r in (0, m - 1):
-        assert np.array_equal(y[r], o.matmul(kind + "_q8", w, xq[r * nb:(r + 1) * nb], n_out, n_in), equal_nan=True)
+        assert same_bits(y[r], o.matmul(kind + "_q8", w, xq[r * nb:(r + 1) * nb], n_out, n_in))
 
 
 @pytest.mark.parametrize("kind", QUANT_TYPES)
@@ -74,6 +70,20 @@ def test_scales_that_are_not_finite(o, h, kind, m, n_out):
 
 
 @pytest.mark.parametrize("kind", QUANT_TYPES)
+@pytest.mark.parametrize("m,n_out", [(65, 96), (128, 5632)])
+def test_scales_at_the_ends_of_the_half_range(o, h, kind, m, n_out):
+    """Subnormal and largest half scales on both sides, and zero weights under negative scales."""
+    n_in = 320
+    w, xq = inputs(o, kind, m, n_out, n_in, seed=4)
+    nb = n_in // 32
+    rng = np.random.default_rng(5)
+    w["d"] = rng.choice(np.array([0x0001, 0x8001, 0x03ff, 0x0400, 0x7bff, 0xfbff, 0x8000, 0x2c00], np.uint16), len(w))
+    xq["d"] = rng.choice(np.array([0x0001, 0x03ff, 0x7bff, 0x0000, 0x2c00], np.uint16), len(xq))
+    w["qs"][7 * nb:8 * nb] = 0 if kind != "q4_0" else 0x88
+    check(o, h, kind, w, xq, m, n_out, n_in)
+
+
+@pytest.mark.parametrize("kind", QUANT_TYPES)
 @pytest.mark.parametrize("m,n_in,n_ff", [(33, 320, 4096), (65, 576, 160), (130, 896, 4864), (257, 1600, 6560)])
 def test_swiglu_tiles_bit_exact(o, h, kind, m, n_in, n_ff):
     """gate|up with the product and its blocks in the epilogue against the separate entries, at both
@@ -88,5 +98,5 @@ def test_swiglu_tiles_bit_exact(o, h, kind, m, n_in, n_ff):
     dg, du, dx = (H.DeviceBuffer.of(a) for a in (wg, wu, xq))
     out, outq = H.DeviceBuffer(m * n_ff * 4), H.DeviceBuffer(m * n_ff // 32 * 34)
     H.call("matmul_q8_swiglu", C.c_int(t), dx, m, n_in, dg, du, n_ff, out, outq)
-    assert same(out.download(np.float32), want)
+    assert same_bits(out.download(np.float32), want)
     assert outq.download(np.uint8).tobytes() == h.quantize_row_q8_0(want).tobytes()
