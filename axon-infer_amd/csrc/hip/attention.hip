@@ -729,8 +729,8 @@ bool launch_block(const AttnArgs& a, uint32_t n_rows) {
 // multiplies (an MFMA costs about what four of them do) but their operands: a broadcast of pairs is
 // an operand modifier, where a multiply took it from LDS (one 16-byte read per pair and 4 positions)
 // or from a scalar register (v_mul_f32 with one issues at half rate). So LDS holds little but the
-// scores, and a workgroup keeps 32 pairs at up to 1088 positions, or 16 at 2176, where the blocked
-// kernel above falls back to one row at a time from about 1000.
+// scores, and a workgroup keeps 32 pairs at up to 1024 positions, or 16 at 2112 (1152 and 2304 with an
+// fp16 cache), where the blocked kernel above falls back to one row at a time from about 1000.
 //   scores   K tiles of 64 positions x 32 dims go through a ring of three 8 KB stages by LDS-DMA
 //            (16-byte chunks XOR-swizzled, so that the lanes' row reads spread over the banks);
 //   softmax  each wave its own four pairs: max, exp, the fused kernel's 256-thread double-sum tree
@@ -753,7 +753,7 @@ __host__ __device__ constexpr uint32_t stage_bytes_of() { return F16 ? 4096 : 81
 __host__ __device__ inline uint32_t tile_pitch(uint32_t max_vis) { return ((max_vis + 63) & ~63u) + 16; }
 
 template <uint32_t G, uint32_t R>
-__host__ __device__ constexpr uint32_t tile_waves() { return (G * R + 3) / 4; }
+__host__ __device__ constexpr uint32_t tile_waves() { return G * R / 4; }
 
 template <bool F16, uint32_t G, uint32_t R>
 __host__ __device__ inline size_t tile_lds(uint32_t max_vis) {
@@ -786,21 +786,14 @@ __device__ __forceinline__ void products_ahead() {
   __builtin_amdgcn_sched_group_barrier(0x2, 8, 0);
 }
 
-template <int I, int N, typename F>
-__device__ __forceinline__ void for_each_index(F f) {
-  if constexpr (I < N) {
-    f.template operator()<I>();
-    for_each_index<I + 1, N>(f);
-  }
-}
-
 // (Four waves per SIMD: two workgroups of 32 pairs share a CU as long as their LDS allows it, up to
 // about 400 positions. With 189 registers for the fp16 cache, which the direct loads once took, it was
 // one: 270 rows of 32 / 8 heads behind 218 positions 61 -> 55.5 us, 56 in the blocked kernel. The 16-pair
 // form is taken where its LDS leaves one workgroup per CU anyway.)
 template <bool F16, uint32_t G, uint32_t R>
 __global__ __launch_bounds__((64 * tile_waves<G, R>()), (G * R == 32 ? 4 : 2)) void attention_tile_kernel(AttnArgs a, uint32_t n_rows) {
-  constexpr uint32_t kPairs = G * R, W = tile_waves<G, R>();
+  static_assert(G % 4 == 0, "a wave's pairs belong to one row");
+  constexpr uint32_t W = tile_waves<G, R>();
   constexpr uint32_t es = F16 ? 2 : 4;
   constexpr uint32_t kStage = stage_bytes_of<F16>();
   constexpr uint32_t kCopies = kStage / 1024;  // 1 KB copies per stage
@@ -834,13 +827,15 @@ __global__ __launch_bounds__((64 * tile_waves<G, R>()), (G * R == 32 ? 4 : 2)) v
   auto aligned = [&](int64_t off) { return ((base + static_cast<uintptr_t>(off) * es) & 15u) == 0; };
   shared = shared && aligned(k_off[0]) && aligned(v_off[0]);
 
-  // Pair 4 wave + v of this wave: its row within the block (R for none) and its positions.
+  // Pair 4 wave + v of this wave: its row within the block and its positions. (All four have the same: the
+  // per-pair tests below are uniform. They stand: without them the compiler schedules the adds of a half
+  // together with the store of its scores, and 200 registers spill.)
   uint32_t prow[4], pvis[4], wmax = 0;
   uint32_t wmin = 0xffffffffu;  // positions that all of the wave's pairs see
 #pragma unroll
   for (uint32_t v = 0; v < 4; ++v) {
     const uint32_t pr = 4 * wave + v;
-    prow[v] = pr < kPairs ? pr / G : R;
+    prow[v] = pr / G;
     pvis[v] = 0;
 #pragma unroll
     for (uint32_t i = 0; i < R; ++i) pvis[v] = prow[v] == i ? nv[i] : pvis[v];
@@ -882,7 +877,7 @@ __global__ __launch_bounds__((64 * tile_waves<G, R>()), (G * R == 32 ? 4 : 2)) v
   // This lane's part of the pairs' queries: lane 4 b + i of register k holds dim 16 k + b of pair i.
   float qa[4];
   {
-    const uint32_t pr = min(4 * wave + (lane & 3u), kPairs - 1);
+    const uint32_t pr = 4 * wave + (lane & 3u);
     const uint32_t r = min(r0 + pr / G, n_rows - 1);
     const float* q = a.q + static_cast<size_t>(r) * a.q_stride + static_cast<size_t>(g * G + pr % G) * 64 + (lane >> 2);
 #pragma unroll

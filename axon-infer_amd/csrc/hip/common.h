@@ -280,6 +280,21 @@ __device__ __forceinline__ int32_t dot32(const int32_t (&a)[8], const int32_t (&
   return s;
 }
 
+// f.operator()<I>(), <I + 1>, ... <N - 1>: a loop whose index is a constant.
+template <int I, int N, typename F>
+__device__ __forceinline__ void for_each_index(F f) {
+  if constexpr (I < N) {
+    f.template operator()<I>();
+    for_each_index<I + 1, N>(f);
+  }
+}
+
+// The value that lane L of this lane's row of 16 holds.
+template <int L>
+__device__ __forceinline__ float row_lane(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x150 + L, 0xf, 0xf, true));  // row_newbcast
+}
+
 // ------------------------------------------------------------------------------------------
 // Reductions over lanes.
 

@@ -41,20 +41,6 @@ __device__ __forceinline__ float weight_value(uint32_t bits) {
   else return bf16_bits_to_float(bits);
 }
 
-// The value that lane L of this lane's row of 16 holds.
-template <int L>
-__device__ __forceinline__ float row_lane(float x) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x150 + L, 0xf, 0xf, true));  // row_newbcast
-}
-
-template <int I, int N, typename F>
-__device__ __forceinline__ void for_each_index(F f) {
-  if constexpr (I < N) {
-    f.template operator()<I>();
-    for_each_index<I + 1, N>(f);
-  }
-}
-
 // W waves of 4 activation rows. PAIR: the weight rows' elements can be loaded two at a time.
 template <int T, uint32_t W, bool PAIR>
 __global__ __launch_bounds__(64 * W) void matmul_float_kernel(const uint8_t* __restrict__ w, const float* __restrict__ x,

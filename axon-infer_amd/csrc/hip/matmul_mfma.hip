@@ -10,17 +10,20 @@
 //   acc += float(sumi) * d_w * d_x                      (Q8_0, Q4_0: sumi includes the -8 offset)
 //   acc += float(sumi) * d_w * d_x + m_w * d_x * float(sumx)          (Q4_1)
 //
-// so every output is bit-identical to the scalar table's. Q4 nibbles enter the MFMA as
-// unsigned values 0..15; the Q4_0 offset is applied as -8 * sum(qx) in int32.
+// so every output is bit-identical to the scalar table's.
 //
-// Workgroup tile: 64 activation rows x 64 weight rows (four waves, 16 weight rows each, four
-// 16-row activation tiles per wave), K staged through LDS 16 blocks at a time.
+//  * mfma_q8_kernel, described here, takes any block count and alignment: Q4 nibbles enter the MFMA as
+//    unsigned values 0..15, the Q4_0 offset is applied as -8 * sum(qx) in int32. A workgroup owns 64
+//    activation rows x 64 weight rows (four waves, 16 weight rows each, four 16-row activation tiles
+//    per wave), K staged through LDS 16 blocks at a time.
+//  * Rows of whole dwords run mfma_rows_kernel (3 to 64 rows in 16-row tiles), mfma_tile_kernel (up to
+//    32 rows of wide matrices) or mfma_wide_kernel (more rows: 32 x 32 or 16 x 16 sums, Q4_0 nibbles as
+//    16 (q - 8), sums accumulated onto the bits of a float). Each says below what it does otherwise.
 #include "common.h"
 #include "matvec.h"
 #include "wide_tiles.h"
 
 #include <type_traits>
-#include <utility>
 
 namespace axon_hip {
 
@@ -781,19 +784,6 @@ __device__ __forceinline__ float scaled_sum(int32_t biased, float dw, float bias
 
 __device__ __forceinline__ bool half_not_finite(uint32_t h) { return (h & 0x7c00u) == 0x7c00u; }
 
-template <typename F, int... I>
-__device__ __forceinline__ void static_for_each(F f, std::integer_sequence<int, I...>) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F f) { static_for_each(f, std::make_integer_sequence<int, N>{}); }
-
-// The value that lane L of this lane's row of 16 holds.
-template <int L>
-__device__ __forceinline__ float row_lane(float x) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x150 + L, 0xf, 0xf, true));  // row_newbcast
-}
-
 template <int T>
 __host__ __device__ constexpr uint32_t pair_dwords() { return (2 * block_bytes<T>() + 3) / 4; }
 
@@ -961,7 +951,7 @@ __global__ __launch_bounds__(kThreads, 2) void mfma_wide_kernel(MatvecArgs args)
           int32_t sum = 0;
 #pragma unroll
           for (uint32_t j = 0; j < 8; ++j) sum = __builtin_amdgcn_sdot4(static_cast<int32_t>(q[j]), 0x01010101, sum, false);
-          xs[b * XP + row] = dx * static_cast<float>(sum);  // exact, as in mfma_tile_kernel
+          xs[b * XP + row] = dx * static_cast<float>(sum);  // exact: 11 bits times at most 13
         }
       }
     }
@@ -1128,8 +1118,8 @@ __global__ __launch_bounds__(kThreads, 2) void mfma_wide_kernel(MatvecArgs args)
       const float d = amax / 127.0f;
       const float id = d != 0.0f ? 1.0f / d : 0.0f;
       const uint32_t dh = float_to_half_bits(d);
-      static_for<ND>([&](auto vc) {
-        constexpr uint32_t v = vc.value;
+      for_each_index<0, ND>([&]<int I>() {
+        constexpr uint32_t v = I;
         const uint32_t rr = row_of(v);
         const uint32_t dv = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(dh), 0x150 + v, 0xf, 0xf, true));
         uint8_t* blk = args.outq + (static_cast<size_t>(m0 + rr) * row_blocks + (n0 + n) / kQK) * kBytesQ8_0;

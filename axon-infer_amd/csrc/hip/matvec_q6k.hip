@@ -477,14 +477,6 @@ __device__ __forceinline__ void planar_fetch_half(const uint8_t* col, uint32_t n
   b.d = reinterpret_cast<const uint16_t*>(col + static_cast<size_t>(208) * n_out)[row];
 }
 
-template <int I, int N, typename F>
-__device__ __forceinline__ void for_each_index(F f) {
-  if constexpr (I < N) {
-    f.template operator()<I>();
-    for_each_index<I + 1, N>(f);
-  }
-}
-
 template <uint32_t S>
 __global__ __launch_bounds__(256, 2) void q6k_planar_mfma_kernel(MatvecArgs args, uint32_t n_in, size_t col_bytes,
                                                                  uint32_t m_total) {
