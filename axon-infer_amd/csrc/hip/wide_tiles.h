@@ -4,7 +4,7 @@
 // round costs nearly a whole one however few workgroups it holds. So the tile is the one of the least
 // estimated time: rounds times blocks per row times the time of a block, plus what a round costs
 // whatever its blocks. With fixed numbers of workgroups as lines (512 for the largest and the 32 x 64
-// tiles, 320 for 64 x 64), Q8_0 174 x 4168 x 1984 ran 786 workgroups of 32 x 32 in 21.4 us where 198 of
+// tiles, 320 for 64 x 64), Q8_0 174 x 4168 x 1984 ran 786 workgroups of 32 x 32 in 21.5 us where 198 of
 // 64 x 64 take 20.1 and 396 of 32 x 64 19.2; Q4_0 300 x 3606 x 5760 570 of 32 x 64 in 72 us where 285 of
 // 64 x 64 take 55.5.
 // Fitted to 655 shapes (33 to 512 rows, 400 to 32768 outputs, 64 to 8192 inputs) on an MI355X: 0.5 % off
