@@ -20,9 +20,13 @@
 // F16, us: one lane walking its row in memory -> both operands in LDS, a thread one output of one
 // row -> now: 2048 x 2048 at 16 rows 252 -> 29 -> 16.5, at one row 237 -> 27 -> 15.8.
 //
-// matmul_blocks_kernel (Q8_0 / Q4_0 / Q4_1): one lane per output, whose short rows of blocks the L1
-// holds (2048 x 2048 at 16 rows 35-47 us); staged as above it ran 34-36 us at 16 rows, and slower
-// from 17 on.
+// matmul_lane_kernel: one lane per output, for Q8_0 / Q4_0 / Q4_1, whose short rows of blocks the L1
+// holds (2048 x 2048 at 16 rows 35-47 us; staged as above it ran 34-36 us at 16 rows, and slower from 17
+// on), and for float weights in very short rows, of which a workgroup above holds 16 in a chunk of 256
+// elements. Where the line lies, us, a lane per output / tiles: F16 at 300 rows, 30000 outputs, 14 elements
+// 105 / 103, 16 246 / 102 (F32: 9 elements 88 / 117, 12 152 / 100); at 8 rows, 40000 outputs, 26 elements 15.8 /
+// 15.7, 32 21.2 / 15.7 (12000 outputs 8.6 / 6.6); at one row, 9000 outputs, 49 elements 6.1 / 7.0, 56 9.0 / 6.4,
+// 32000 outputs, 64 elements 11.0 / 13.2, 110000 outputs, 16 elements 5.3 / 36.6.
 #include "common.h"
 #include "matmul_float.h"
 
@@ -230,7 +234,12 @@ int matmul_float_tiles(const uint8_t* w, const float* x, float* y, uint32_t n_ro
 template <int T>
 __device__ float row_dot(const uint8_t* w, const float* x, uint32_t n_in) {
   float acc = 0.0f;
-  if constexpr (T == Q8_0) {
+  if constexpr (T == F32 || T == F16 || T == BF16) {
+    for (uint32_t i = 0; i < n_in; ++i) {
+      if constexpr (T == F32) acc += reinterpret_cast<const float*>(w)[i] * x[i];
+      else acc += weight_value<T>(reinterpret_cast<const uint16_t*>(w)[i]) * x[i];
+    }
+  } else if constexpr (T == Q8_0) {
     for (uint32_t b = 0; b < n_in / kQK; ++b) {
       const uint8_t* blk = w + b * kBytesQ8_0;
       const float d = half_bits_to_float(*reinterpret_cast<const uint16_t*>(blk));
@@ -265,7 +274,7 @@ __device__ float row_dot(const uint8_t* w, const float* x, uint32_t n_in) {
 }
 
 template <int T>
-__global__ __launch_bounds__(256) void matmul_blocks_kernel(const uint8_t* __restrict__ w, const float* __restrict__ x,
+__global__ __launch_bounds__(256) void matmul_lane_kernel(const uint8_t* __restrict__ w, const float* __restrict__ x,
                                                            float* __restrict__ y, uint32_t n_rows, uint32_t n_out,
                                                            uint32_t n_in, uint32_t y_stride, size_t row_bytes) {
   const uint32_t o = blockIdx.x * blockDim.x + threadIdx.x;
@@ -292,15 +301,28 @@ int matmul_float_launch(int type, const void* w, const float* x, float* y, uint3
     return fail(kInvalidArgument, "quantized matmul: n_in %u is not a multiple of 32", n_in);
   const dim3 grid(static_cast<uint32_t>(ceil_div(n_out, 256)), n_rows);
   const uint8_t* wb = static_cast<const uint8_t*>(w);
+  // (Rows of 32 bytes apart fall on few channels: 246 us where rows of 30 take 122.)
+  const bool short_rows =
+      n_rows <= 65535 && ((row_bytes <= (type == F32 ? 36 : 28) && row_bytes != 32) || (row_bytes <= 80 && n_rows * row_bytes <= 416) ||
+                          (n_rows == 1 && ((row_bytes <= 100 && n_out >= 8192) || (row_bytes <= 128 && n_out >= 32000))));
+  auto by_lanes = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream(), wb, x, y, n_rows, n_out, n_in, y_stride, row_bytes);
+    return check_launch("matmul_float");
+  };
   switch (type) {
-  case F32: return matmul_float_tiles<F32>(wb, x, y, n_rows, n_out, n_in, y_stride, row_bytes);
-  case F16: return matmul_float_tiles<F16>(wb, x, y, n_rows, n_out, n_in, y_stride, row_bytes);
-  case BF16: return matmul_float_tiles<BF16>(wb, x, y, n_rows, n_out, n_in, y_stride, row_bytes);
-  case Q8_0: hipLaunchKernelGGL(matmul_blocks_kernel<Q8_0>, grid, dim3(256), 0, stream(), wb, x, y, n_rows, n_out, n_in, y_stride, row_bytes); break;
-  case Q4_0: hipLaunchKernelGGL(matmul_blocks_kernel<Q4_0>, grid, dim3(256), 0, stream(), wb, x, y, n_rows, n_out, n_in, y_stride, row_bytes); break;
-  default: hipLaunchKernelGGL(matmul_blocks_kernel<Q4_1>, grid, dim3(256), 0, stream(), wb, x, y, n_rows, n_out, n_in, y_stride, row_bytes); break;
+  case F32:
+    if (short_rows) return by_lanes(matmul_lane_kernel<F32>);
+    return matmul_float_tiles<F32>(wb, x, y, n_rows, n_out, n_in, y_stride, row_bytes);
+  case F16:
+    if (short_rows) return by_lanes(matmul_lane_kernel<F16>);
+    return matmul_float_tiles<F16>(wb, x, y, n_rows, n_out, n_in, y_stride, row_bytes);
+  case BF16:
+    if (short_rows) return by_lanes(matmul_lane_kernel<BF16>);
+    return matmul_float_tiles<BF16>(wb, x, y, n_rows, n_out, n_in, y_stride, row_bytes);
+  case Q8_0: return by_lanes(matmul_lane_kernel<Q8_0>);
+  case Q4_0: return by_lanes(matmul_lane_kernel<Q4_0>);
+  default: return by_lanes(matmul_lane_kernel<Q4_1>);
   }
-  return check_launch("matmul_float");
 }
 
 }  // namespace axon_hip

@@ -42,6 +42,18 @@ def test_float_matmul_tiles(o, h, kind, n_rows, n_out, n_in):
         assert np.array_equal(h.matmul(kind, w, x, n_out, n_in).view(np.uint32), want[:n_out].view(np.uint32))
 
 
+# Either side of the lines between one lane per output and the tiles: 28 bytes a row of 16-bit weights, 36
+# (but 32) of 32-bit ones, 416 bytes in all rows, and 100 or 128 bytes of one row against many outputs.
+@pytest.mark.parametrize("kind", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("n_rows,n_out,n_in", [(40, 300, 7), (40, 300, 8), (40, 300, 9), (40, 300, 10), (33, 270, 14), (33, 270, 15),
+                                               (8, 257, 13), (8, 257, 26), (8, 257, 27), (1, 100, 40), (1, 100, 41), (1, 8192, 50),
+                                               (1, 8191, 50), (1, 32000, 64), (1, 31999, 64), (1, 32001, 65)])
+def test_float_matmul_short_rows(o, h, kind, n_rows, n_out, n_in):
+    w, x = weights(kind, n_out * n_in, 9), random_floats(n_rows * n_in, 10, 3.0)
+    want = o.matmul(kind, w, x, n_out, n_in, n_rows=n_rows, y_stride=n_out + 1)
+    assert same_bits(h.matmul(kind, w, x, n_out, n_in, n_rows=n_rows, y_stride=n_out + 1), want)
+
+
 @pytest.mark.parametrize("kind", ["f32", "f16", "bf16"])
 def test_float_matmul_infinities_stay_in_their_row(o, h, kind):
     n_rows, n_out, n_in = 18, 20, 300
